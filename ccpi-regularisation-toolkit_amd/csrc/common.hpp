@@ -271,33 +271,53 @@ __device__ inline bool solve_stopped(const Ctrl* c) { return c != nullptr && c->
 // ---------------------------------------------------------------------------
 // correctly rounded single-precision square root
 // ---------------------------------------------------------------------------
-// For x in [2^-96, FLT_MAX], v_sqrt_f32 is within one ulp of sqrt(x) and the
-// neighbours r -/+ 1 ulp of its result r are normal and finite; the rounded
-// root is r - 1 ulp when x - (r - 1 ulp) r <= 0, r + 1 ulp when
-// x - (r + 1 ulp) r > 0, and r otherwise (both residuals by fma, exact).
-// This is the selection the compiler's IEEE expansion of sqrtf makes after
-// it has scaled tiny arguments and before it patches zeros and infinities,
-// so on that interval it returns sqrtf's bits (checked over every float of
-// it by cilreg_check_sqrt_rn).  A wave with any lane outside the interval
-// (zero, denormal, negative, infinite, NaN) calls sqrtf.
-//
-// The two decisions are read from the sign bits of (r -/+ 1 ulp) r - x, the
-// negated residuals (an exact zero is +0, so "x - (r - 1 ulp) r <= 0" is a
-// clear sign bit): the root is the bit pattern of r - 1 ulp plus one for
-// each neighbour whose square lies below x (at most r + 1 ulp: the second
-// implies the first).  Integer shifts and one add instead of compares and
-// selects, which on this target wait two cycles each between the compare and
-// its use.
+// For x in [2^-96, FLT_MAX], with t = v_rsq_f32(x) and g = x t, one step
+// g + (x - g^2) t / 2 (both by fused multiply-add) is the correctly rounded
+// root, so on that interval it returns sqrtf's bits (checked over every float
+// by cilreg_check_sqrt_rn).  That is one transcendental and four plain
+// operations (21 issue cycles); sqrtf's expansion scales the argument, takes
+// v_sqrt_f32, selects among three neighbours and patches special values
+// (about 70), and the selection alone took 30.  A wave with any lane outside
+// the interval (zero, denormal, negative, infinite, NaN) calls sqrtf.
+// sqrt_in: the interval is the caller's to guarantee.
+__device__ inline float sqrt_in(float x) {
+    const float t = __builtin_amdgcn_rsqf(x);
+    const float g = x * t;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * t, g);
+}
 __device__ inline float sqrt_rn(float x) {
     const bool fast = x >= 0x1p-96f && x <= 0x1.fffffep127f;   // false for NaN
     if (__builtin_amdgcn_ballot_w64(!fast)) return sqrtf(x);
-    const float r = __builtin_amdgcn_sqrtf(x);
-    const uint32_t ri = __float_as_uint(r);
-    const float rm = __uint_as_float(ri - 1u), rp = __uint_as_float(ri + 1u);
-    const uint32_t above_m = __float_as_uint(__builtin_fmaf(rm, r, -x)) >> 31;   // 1: x - (r - 1 ulp) r > 0
-    const uint32_t above_p = __float_as_uint(__builtin_fmaf(rp, r, -x)) >> 31;   // 1: x - (r + 1 ulp) r > 0
-    return __uint_as_float(ri - 1u + above_m + above_p);
+    return sqrt_in(x);
 }
+
+// ---------------------------------------------------------------------------
+// correctly rounded single-precision reciprocal and quotient
+// ---------------------------------------------------------------------------
+// For y in [2^-125, 2^125], v_rcp_f32 followed by one Newton step (two fused
+// multiply-adds) is the correctly rounded reciprocal r (checked for every
+// such float by cilreg_check_rcp_in), and for a = 0 or 2^-100 <= |a| with
+// 2^-60 <= |y| <= 2^64, |a| <= 2^64 the quotient a / y is a r corrected once
+// by its residual (checked by cilreg_check_div_in; all 2^46 pairs of
+// significands give the IEEE quotient, and in that range every step scales
+// with the exponents exactly).  The residual is negated so that a = -0 keeps
+// its sign.  The compiler's IEEE expansion of a / y (two scalings, v_rcp,
+// five multiply-adds, fmas, fixup) issues in about 49 cycles; rcp_in takes
+// 16 and each quotient of a shared divisor 10 more.
+__device__ inline float rcp_in(float y) {
+    const float r = __builtin_amdgcn_rcpf(y);
+    return __builtin_fmaf(__builtin_fmaf(-y, r, 1.0f), r, r);
+}
+__device__ inline float div_in(float a, float y, float r) {
+    const float q = a * r;
+    return __builtin_fmaf(-__builtin_fmaf(y, q, -a), r, q);
+}
+// The test of a dividend: tiny_key(a) < kTinyKey exactly when 0 < |a| < 2^-100
+// (zero wraps to the largest key), so the smallest key of many dividends
+// decides for all of them.
+constexpr uint32_t kTinyKey = (0x0d800000u << 1) - 1u;   // 2^-100 is 0x0d800000
+__device__ inline uint32_t tiny_key(float a) { return (__float_as_uint(a) << 1) - 1u; }
+__device__ inline uint32_t min_key(uint32_t a, uint32_t b) { return a < b ? a : b; }
 
 // Correctly rounded double square root for x in [2^-1000, 2^1000] (no
 // scaling needed there): an estimate g = x rsq(x), h = rsq(x) / 2, one
@@ -352,6 +372,26 @@ template <> struct Mixed<float> {
         if (__builtin_amdgcn_ballot_w64(!(lo == hi))) r = (float)((double)num / c);
         return r;
     }
+    // N quotients with c = 1 + lt and rc = RN(1 / c) at hand: one test for the
+    // wave that divides.
+    template <int N>
+    __device__ static inline void pd_div_n(float (&v)[N], double c, double rc) {
+        float lo[N];
+        bool odd = false;
+        #pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const double q = (double)v[i] * rc, d = fabs(q) * 0x1p-50;
+            lo[i] = (float)(q - d);
+            odd = odd || !(lo[i] == (float)(q + d));
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0, 0)) {
+            #pragma unroll
+            for (int i = 0; i < N; ++i) v[i] = (float)((double)v[i] / c);
+            return;
+        }
+        #pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = lo[i];
+    }
     // squared minmod, ROF_TV_core.c:132-133.  The reference multiplies in
     // double (fabs promotes) and rounds the product to float; the factor is
     // 0, +-0.5 or +-1, so the double product is exact and its rounding to
@@ -403,6 +443,100 @@ template <> struct Mixed<double> {
         for (int q = 0; q < N; ++q) m[q] = minmod_sq(a[q], b[q]);
     }
 };
+
+// ---------------------------------------------------------------------------
+// projection of a dual point
+// ---------------------------------------------------------------------------
+// P onto the unit ball (iso: P / |P| when |P| > 1, utils.c:184-196) or box
+// (aniso: P_d / max(|P_d|, 1), :197-211).
+//
+// In float the iso form runs without a branch per lane: x = max(|P|^2, 1) is
+// in range of sqrt_in and rcp_in unless |P|^2 overflowed, the factor of a
+// point inside the ball is then 1/sqrt(1) = 1 exactly and leaves P as it is
+// (a NaN |P|^2 gives x = 1 too: the reference does not scale there either).
+// A wave with an infinite |P|^2 takes the reference's expressions.  The box
+// form is the median of (P_d, -1, 1) for finite P_d: P_d / |P_d| is exactly
+// +-1 and P_d / 1 is P_d; a wave with an infinite or NaN P_d divides.
+template <int DIM, typename T, bool ISO>
+__device__ inline void project_unit_ref(T& p1, T& p2, T& p3) {
+    if (ISO) {
+        T n2 = p1 * p1 + p2 * p2;
+        if (DIM == 3) n2 = n2 + p3 * p3;
+        if (n2 > (T)1) {
+            const T s = (T)1 / (T)(sizeof(T) == 4 ? (T)sqrtf((float)n2) : (T)sqrt((double)n2));
+            p1 = p1 * s;
+            p2 = p2 * s;
+            if (DIM == 3) p3 = p3 * s;
+        }
+    } else {
+        T a1 = fabs(p1), a2 = fabs(p2);
+        if (a1 < (T)1) a1 = 1;
+        if (a2 < (T)1) a2 = 1;
+        p1 = p1 / a1;
+        p2 = p2 / a2;
+        if (DIM == 3) {
+            T a3 = fabs(p3);
+            if (a3 < (T)1) a3 = 1;
+            p3 = p3 / a3;
+        }
+    }
+}
+// N points at once: one test for the exceptional wave, so the N projections
+// form one straight line of independent chains.
+template <int DIM, typename T, bool ISO, int N>
+__device__ inline void project_unit_n(T (&p1)[N], T (&p2)[N], T (&p3)[N]) {
+    if constexpr (!std::is_same<T, float>::value) {
+        #pragma unroll
+        for (int i = 0; i < N; ++i) project_unit_ref<DIM, T, ISO>(p1[i], p2[i], p3[i]);
+    } else if constexpr (ISO) {
+        float x[N], top = 1.0f;
+        #pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float n2 = p1[i] * p1[i] + p2[i] * p2[i];
+            if (DIM == 3) n2 = n2 + p3[i] * p3[i];
+            x[i] = __builtin_fmaxf(n2, 1.0f);
+            top = i == 0 ? x[0] : __builtin_fmaxf(top, x[i]);
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(top > 0x1.fffffep127f) != 0, 0)) {
+            #pragma unroll
+            for (int i = 0; i < N; ++i) project_unit_ref<DIM, T, ISO>(p1[i], p2[i], p3[i]);
+            return;
+        }
+        #pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float s = rcp_in(sqrt_in(x[i]));
+            p1[i] = p1[i] * s;
+            p2[i] = p2[i] * s;
+            if (DIM == 3) p3[i] = p3[i] * s;
+        }
+    } else {
+        bool odd = false;
+        #pragma unroll
+        for (int i = 0; i < N; ++i) {
+            odd = odd || !(fabsf(p1[i]) <= 0x1.fffffep127f) || !(fabsf(p2[i]) <= 0x1.fffffep127f);
+            if (DIM == 3) odd = odd || !(fabsf(p3[i]) <= 0x1.fffffep127f);
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0, 0)) {
+            #pragma unroll
+            for (int i = 0; i < N; ++i) project_unit_ref<DIM, T, ISO>(p1[i], p2[i], p3[i]);
+            return;
+        }
+        #pragma unroll
+        for (int i = 0; i < N; ++i) {
+            p1[i] = __builtin_amdgcn_fmed3f(p1[i], -1.0f, 1.0f);
+            p2[i] = __builtin_amdgcn_fmed3f(p2[i], -1.0f, 1.0f);
+            if (DIM == 3) p3[i] = __builtin_amdgcn_fmed3f(p3[i], -1.0f, 1.0f);
+        }
+    }
+}
+template <int DIM, typename T, bool ISO>
+__device__ inline void project_unit(T& p1, T& p2, T& p3) {
+    T a[1] = {p1}, b[1] = {p2}, c[1] = {p3};
+    project_unit_n<DIM, T, ISO>(a, b, c);
+    p1 = a[0];
+    p2 = b[0];
+    p3 = c[0];
+}
 
 template <typename T> __device__ inline T dsqrt(T x);
 template <> __device__ inline float dsqrt<float>(float x) { return sqrt_rn(x); }

@@ -69,7 +69,7 @@ static void launch_fgp2(const Fgp2Args<T, S>& a, bool iso, bool small, hipStream
 // residual (FGP_TV_core.c:66,123).  Iterations run two per pass
 // (fgp2_iter_kernel) unless opts.depth == 1 or, by default, a 2D image has
 // kFgp2dPassMaxPixels or more; an odd last iteration runs on the
-// one-iteration kernel.  P_j lives in buffer
+// one-iteration kernel.  2D images in FP32 arithmetic take fgp_solve_2d.  P_j lives in buffer
 // j mod nbuf (nbuf = 4 with two-iteration passes, which write P_{k+1} and
 // P_{k+2} while reading P_k and P_{k-1}; 3 otherwise).
 template <typename T, typename S>
@@ -80,13 +80,19 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
     *iters_done = 0;
     *re = 0.f;
     if (iter <= 0) return 0;
+    if constexpr (std::is_same<T, float>::value) {
+        // under a scratch limit large images keep the path whose workspace decides what fits
+        if (dim == 2 && opts.depth != 1 && !(opts.scratch && (size_t)nx * ny >= kFgp2dPassMaxPixels))
+            return fgp_solve_2d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, opts, s, iters_done, re, ws);
+    }
     const size_t n = (size_t)nx * ny * nz;
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T) > sizeof(S) ? sizeof(T) : sizeof(S));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;
     const bool iso = method == 0;
     // returning the state after a stop needs the stop iteration's own pass
     const bool pass2 = opts.depth == 2 || (opts.depth == 0 && (dim == 3 || n < kFgp2dPassMaxPixels));
-    const int width = (pass2 && iter > 1 && !(ws && epsil != (T)0)) ? 2 : 1;
+    const bool two = pass2 && iter > 1 && !(ws && epsil != (T)0);
+    const int width = (two && (dim == 3 || std::is_same<T, double>::value)) ? 2 : 1;
     // 2D two-iteration passes: 64 x 4 tiles unless 8 rows are asked for
     const int ty2d = opts.tile_y == 8 ? 8 : 4;
     Geom g;
@@ -105,7 +111,7 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
         g = plan_geom(small ? fgp_kernel_ptr<3, 4, T, S, uint32_t>(iso) : fgp_kernel_ptr<3, 4, T, S, uint64_t>(iso),
                       TX * 4, nx, ny, nz, 4, opts.zchunk);
 
-    const int nbuf = width == 2 ? 4 : 3;
+    const int nbuf = two ? 4 : 3;
     Arena ar;
     if (opts.scratch) ar.use_external(opts.scratch, opts.scratch_bytes);   // the allocation-free entry point
     size_t oP[4][3], oD[2], oCtrl, oPart;
@@ -217,8 +223,10 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
             a.ctrl = ctrl;
             a.g = g;
             if (dim == 2) {
-                if (ty2d == 8) launch_fgp2<8, T, S, 2>(a, iso, small, s);
-                else launch_fgp2<4, T, S, 2>(a, iso, small, s);
+                if constexpr (std::is_same<T, double>::value) {
+                    if (ty2d == 8) launch_fgp2<8, T, S, 2>(a, iso, small, s);
+                    else launch_fgp2<4, T, S, 2>(a, iso, small, s);
+                }
             } else if (ty == 8) {
                 launch_fgp2<8>(a, iso, small, s);
             } else {

@@ -268,6 +268,16 @@ __global__ __launch_bounds__(256) void finalize2_kernel(const double* p0, const 
     finalize2_body(p0, p1, nblocks, ctrl, epsil, iter);
 }
 
+// Several checks of one pass in one launch: finalize_body's rule in iteration
+// order (each returns at once after a stop).
+__global__ __launch_bounds__(256) void finalize_n_kernel(const double* partials, int nblocks, Ctrl* ctrl, float epsil,
+                                                         int first, int every, int checks) {
+    for (int c = 0; c < checks; ++c) {
+        finalize_body(partials + 2 * (size_t)c * nblocks, nblocks, ctrl, epsil, first + c * every);
+        __syncthreads();   // the control block and the LDS sums before the next check
+    }
+}
+
 __global__ void ctrl_reset_kernel(Ctrl* ctrl) {
     if (threadIdx.x == 0) {
         ctrl->stopped = 0;
@@ -303,6 +313,12 @@ void launch_finalize(const double* partials, int nblocks, Ctrl* ctrl, float epsi
 void launch_finalize2(const double* p0, const double* p1, int nblocks, Ctrl* ctrl, float epsil, int iter,
                       hipStream_t s) {
     hipLaunchKernelGGL(finalize2_kernel, dim3(1), dim3(256), 0, s, p0, p1, nblocks, ctrl, epsil, iter);
+}
+
+void launch_finalize_n(const double* partials, int nblocks, Ctrl* ctrl, float epsil, int first, int every, int checks,
+                       hipStream_t s) {
+    hipLaunchKernelGGL(finalize_n_kernel, dim3(1), dim3(256), 0, s, partials, nblocks, ctrl, epsil, first, every,
+                       checks);
 }
 
 void launch_ctrl_reset(Ctrl* ctrl, hipStream_t s) {

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdint.h>
+#include <utility>
 #include <vector>
 #include <math.h>
 #include "common.hpp"
@@ -177,6 +178,11 @@ void launch_finalize(const double* partials, int nblocks, Ctrl* ctrl, float epsi
 // with the result of two launch_finalize calls in a row.
 void launch_finalize2(const double* p0, const double* p1, int nblocks, Ctrl* ctrl, float epsil, int iter,
                       hipStream_t s);
+// The rule for `checks` iterations first, first + every, ... in one launch:
+// check c's nblocks partial pairs start at partials + 2 c nblocks; the state
+// is that of `checks` launch_finalize calls in a row.
+void launch_finalize_n(const double* partials, int nblocks, Ctrl* ctrl, float epsil, int first, int every, int checks,
+                       hipStream_t s);
 // Zero the control block (a small fill kernel, safe under graph capture).
 void launch_ctrl_reset(Ctrl* ctrl, hipStream_t s);
 // Fill a float/double/16-bit array with zeros, or copy one array to another.
@@ -257,19 +263,16 @@ Geom plan_geom(K kernel, int threads, int nx, int ny, int nz, int ty, int zc_hin
     return make_geom(nx, ny, nz, ty, (nz + chunks - 1) / chunks);
 }
 
-// Drives `iter` iterations on stream s in passes.  step(k, nk, check0,
-// check1) launches the pass that advances iterations k .. k+nk-1 (nk is 1 or,
-// when the caller's pass width is 2 and two iterations remain, 2); check0 /
-// check1 say whether iteration k / k+1 evaluates the stopping rule, and the
-// pass leaves those residual sums in partials0 / partials1.  drive_passes then
-// launches the finalisers in iteration order, polls the stop flag every
-// opts.poll iterations without draining the queue, and on return has
-// synchronised the stream and filled *iters_done and *re.  With opts.profile
-// every pass is timed with HIP events; the profile reports time per
-// iteration (pass time / nk).
-template <class StepFn>
-int drive_passes(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctrl, double* d_partials0,
-                 double* d_partials1, int nblocks, hipStream_t s, StepFn&& step, int* iters_done, float* re) {
+// The pass loop of every solve: pass(k, nk) launches the pass that advances
+// iterations k .. k+nk-1 (nk = width, fewer in the last pass) and returns what
+// fin needs to launch its finalisers.  Polls the stop flag every opts.poll
+// iterations without draining the queue; on return has synchronised the
+// stream and filled *iters_done and *re.  With opts.profile every pass is
+// timed with HIP events (the finalisers excluded); the profile reports time
+// per iteration (pass time / nk).
+template <class PassFn, class FinFn>
+int drive_core(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctrl, hipStream_t s, PassFn&& pass,
+               FinFn&& fin, int* iters_done, float* re) {
     PinnedCtrl pin;
     const bool use_tol = epsil != 0.0f;
     const bool polls = use_tol && !opts.scratch;   // an allocation-free solve does not poll
@@ -292,23 +295,16 @@ int drive_passes(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctr
     }
     int npass = 0;
     for (int k = 0; k < iter && rc == 0;) {
-        const int nk = (width >= 2 && k + 1 < iter) ? 2 : 1;
-        const bool c0 = use_tol && (k % opts.check_every == 0);
-        const bool c1 = nk == 2 && use_tol && ((k + 1) % opts.check_every == 0);
+        const int nk = iter - k < width ? iter - k : width;
         if (opts.profile) (void)hipEventRecord(pev[2 * npass], s);
-        step(k, nk, c0, c1);
+        const auto checks = pass(k, nk);
         if (opts.profile) {
             (void)hipEventRecord(pev[2 * npass + 1], s);
             pass_k.push_back(k);
             pass_n.push_back(nk);
         }
         ++npass;
-        if (c0 && c1) {
-            launch_finalize2(d_partials0, d_partials1, nblocks, d_ctrl, epsil, k, s);
-        } else {
-            if (c0) launch_finalize(d_partials0, nblocks, d_ctrl, epsil, k, s);
-            if (c1) launch_finalize(d_partials1, nblocks, d_ctrl, epsil, k + 1, s);
-        }
+        fin(checks);
         k += nk;
         since_poll += nk;
         if (polls && since_poll >= opts.poll && k < iter) {
@@ -366,6 +362,61 @@ int drive_passes(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctr
     *iters_done = c.stopped ? c.stop_iter : iter;
     *re = c.re;
     return 0;
+}
+
+// Drives `iter` iterations on stream s in passes of one or two.  step(k, nk,
+// check0, check1) launches the pass that advances iterations k .. k+nk-1
+// (nk is 1 or, when the caller's pass width is 2 and two iterations remain,
+// 2); check0 / check1 say whether iteration k / k+1 evaluates the stopping
+// rule, and the pass leaves those residual sums in partials0 / partials1;
+// the finalisers are launched in iteration order.
+template <class StepFn>
+int drive_passes(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctrl, double* d_partials0,
+                 double* d_partials1, int nblocks, hipStream_t s, StepFn&& step, int* iters_done, float* re) {
+    const bool use_tol = epsil != 0.0f;
+    struct Checks { int k; bool c0, c1; };
+    auto pass = [&](int k, int nk) {
+        const bool c0 = use_tol && (k % opts.check_every == 0);
+        const bool c1 = nk == 2 && use_tol && ((k + 1) % opts.check_every == 0);
+        step(k, nk, c0, c1);
+        return Checks{k, c0, c1};
+    };
+    auto fin = [&](const Checks& c) {
+        if (c.c0 && c.c1) {
+            launch_finalize2(d_partials0, d_partials1, nblocks, d_ctrl, epsil, c.k, s);
+        } else {
+            if (c.c0) launch_finalize(d_partials0, nblocks, d_ctrl, epsil, c.k, s);
+            if (c.c1) launch_finalize(d_partials1, nblocks, d_ctrl, epsil, c.k + 1, s);
+        }
+    };
+    return drive_core(iter, width >= 2 ? 2 : 1, epsil, opts, d_ctrl, s, pass, fin, iters_done, re);
+}
+
+// Passes of up to `width` iterations with any number of checks in them:
+// step(k, nk, mask) launches the pass that advances iterations k .. k+nk-1,
+// bit i of mask set when iteration k+i is checked; the pass leaves the sums
+// of its c-th check in partials + 2 c nblocks.  A stop at iteration j leaves
+// *iters_done = j (the later passes return at once).
+template <class StepFn>
+int drive_deep(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctrl, double* d_partials, int nblocks,
+               hipStream_t s, StepFn&& step, int* iters_done, float* re) {
+    const bool use_tol = epsil != 0.0f;
+    auto pass = [&](int k, int nk) {
+        unsigned mask = 0;
+        int first = -1, checks = 0;
+        for (int i = 0; use_tol && i < nk; ++i)
+            if ((k + i) % opts.check_every == 0) {
+                mask |= 1u << i;
+                if (first < 0) first = k + i;
+                ++checks;
+            }
+        step(k, nk, mask);
+        return std::make_pair(first, checks);
+    };
+    auto fin = [&](std::pair<int, int> c) {
+        if (c.second) launch_finalize_n(d_partials, nblocks, d_ctrl, epsil, c.first, opts.check_every, c.second, s);
+    };
+    return drive_core(iter, width, epsil, opts, d_ctrl, s, pass, fin, iters_done, re);
 }
 
 // One iteration per pass: step(k, check) launches iteration k.

@@ -39,4 +39,20 @@ template <typename T>
 int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsil, T eta, int method, int nonneg,
               int nx, int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re);
 
+// 2D solves with many iterations per launch (opts.depth: 0 = as many as pay,
+// 2 = two; S: storage of the dual fields).
+template <typename S>
+int fgp_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float epsil, int method, int nonneg, int nx,
+                 int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws);
+template <typename S>
+int pd_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float epsil, float lipschitz, int method,
+                int nonneg, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re,
+                const WarmState* ws);
+template <typename S>
+int tgv_solve_2d(const float* d_f, float* d_out, float lambda, float alpha1, float alpha0, int iter, float L2,
+                 float epsil, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re,
+                 const WarmState* ws);
+int rof_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float tau, float epsil, int nx, int ny,
+                 const Opts& opts, hipStream_t s, int* iters_done, float* re);
+
 }  // namespace cilreg

@@ -43,7 +43,8 @@ typedef struct cilreg_opts {
     int profile;         /* 1: time every iteration's kernels with HIP events (see cilreg_last_profile) */
     int wide_index;      /* 1: force 64-bit element indexing (chosen automatically for fields >= 2 GiB) */
     int stream_launches; /* batch: 1 = launch directly instead of capturing one hipGraph */
-    int temporal_depth;  /* iterations fused per pass where supported (FGP, PD, TGV 3D): 0 = auto (2), 1 = off */
+    int temporal_depth;  /* iterations fused per pass where supported: 0 = auto (3D FGP, PD, TGV: 2; 2D: up to 8),
+                            1 = off, 2 = two */
     int autotune;        /* 1: tile_y / zchunk / temporal_depth left at 0 are chosen by cilreg_autotune */
     int persistent;      /* batch: 1 = one persistent work-queue kernel per method group; disabled in this
                             build (cilreg_batch_run returns -1 with the reason) */
@@ -194,6 +195,12 @@ CILREG_API int cilreg_check_sqrt_rn(unsigned long long *mismatches, unsigned lon
  * of differing results (0 expected) and of values checked.  No counterpart in
  * the reference. */
 CILREG_API int cilreg_check_rof_sqrt_d(double eps, unsigned long long *mismatches, unsigned long long *checked);
+/* Self-checks: the kernels' in-range reciprocal against 1 / y for every float
+ * y in [2^-125, 2^125], and their in-range quotient against a / y for every
+ * significand of y with every stride-th significand of a (stride 1: all 2^46
+ * pairs, some 20 seconds).  Counts the differing values and all checked ones. */
+CILREG_API int cilreg_check_rcp_in(unsigned long long *mismatches, unsigned long long *checked);
+CILREG_API int cilreg_check_div_in(unsigned stride, unsigned long long *mismatches, unsigned long long *checked);
 
 /* Achievable HBM bandwidth of the current device, from streaming kernels
  * over arrays of `bytes` each (>= 1 MiB), the mean of `reps` timed launches:
