@@ -82,6 +82,11 @@ int pd_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, T lipschitz, i
         CILREG_CK(hipStreamSynchronize(s));
         return 0;
     }
+    if constexpr (std::is_same<T, float>::value) {
+        if (dim == 2 && opts.depth != 1 && nx > 1 && ny > 1)
+            return pd_solve_2d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, opts, s, iters_done,
+                                  re, ws);
+    }
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T) > sizeof(S) ? sizeof(T) : sizeof(S));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;
     const bool iso = method == 0;
