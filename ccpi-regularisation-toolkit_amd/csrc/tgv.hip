@@ -80,6 +80,11 @@ int tgv_solve(const T* d_f, T* d_out, T lambda, T alpha1, T alpha0, int iter, T 
         CILREG_CK(hipStreamSynchronize(s));
         return 0;
     }
+    if constexpr (std::is_same<T, float>::value) {
+        if (dim == 2 && opts.depth != 1)
+            return tgv_solve_2d<S>(d_f, d_out, lambda, alpha1, alpha0, iter, L2, epsil, nx, ny, opts, s, iters_done, re,
+                                   ws);
+    }
     const int nq = dim == 3 ? 6 : 3;
     // state in FP32 or 16-bit storage lives in pair fields (two channels side by side, tgv_pairs)
     const bool pairs = tgv_pairs<3, S>();
