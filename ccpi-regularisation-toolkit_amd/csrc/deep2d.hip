@@ -1,5 +1,6 @@
-// deep2d.hip -- the shape and width of a 2D method's passes.
+// deep2d.hip -- the shape and width of a 2D or 3D method's passes.
 #include "deep2d.hpp"
+#include "deep3d.hpp"
 
 namespace cilreg {
 
@@ -23,6 +24,38 @@ DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[
             if (us < best_us) {
                 best_us = us;
                 best = DeepPlan{s, w, g};
+            }
+        }
+    }
+    return best;
+}
+
+// Time of a pass: rounds of resident workgroups, each marching its chunk and the
+// planes it repeats at the chunk's ends, one step per plane.
+Deep3Plan plan_deep3(int nx, int ny, int nz, int rlo, int rhi, const Deep3Cost (&cost)[kDeep3Shapes], size_t bytes,
+                     int most, int zchunk) {
+    constexpr double kCacheBytes = 200e6, kLaunchUs = 4.0;
+    const bool stream = (double)bytes * nx * ny * nz > kCacheBytes;
+    Deep3Plan best{};
+    double best_us = 1e300;
+    for (int s = 0; s < kDeep3Shapes; ++s) {
+        const Deep3Shape& sh = kDeep3Shapes_[s];
+        const int h = sh.nw * sh.r;
+        for (int t = 1; t <= most && t <= kDeep3Max; ++t) {
+            const int lo = rlo * t, hi = rhi * t;
+            if (h - lo - hi < 4) break;
+            const long long regions = make_deep3(nx, ny, nz, 64, h, lo, hi, nz).nblocks;
+            const double step = stream ? cost[s].stream_us[t - 1] : cost[s].cached_us[t - 1];
+            for (int c = 1; c <= nz; ++c) {
+                const int zc = zchunk > 0 ? zchunk : (nz + c - 1) / c;
+                const int n = (nz + zc - 1) / zc;
+                const double rounds = (double)((regions * n + sh.slots - 1) / sh.slots);
+                const double us = (kLaunchUs + rounds * step * (zc + (n > 1 ? lo + hi : t))) / t;
+                if (us < best_us * (1 - 1e-9)) {
+                    best_us = us;
+                    best = Deep3Plan{s, t, make_deep3(nx, ny, nz, 64, h, lo, hi, zc)};
+                }
+                if (zchunk > 0) break;
             }
         }
     }

@@ -86,8 +86,9 @@ struct DeepPos {
     int ylo, yhi;      // image rows [ylo, yhi) are stored by this region
     int lin;
 
-    __device__ inline DeepPos(const Deep2D& g) {
-        lin = xcd_logical_block((int)blockIdx.x, g.nblocks);
+    __device__ inline DeepPos(const Deep2D& g) : DeepPos(g, xcd_logical_block((int)blockIdx.x, g.nblocks)) {}
+    __device__ inline DeepPos(const Deep2D& g, int logical) {
+        lin = logical;
         nx = g.nx;
         ny = g.ny;
         const int ty = lin / g.tiles_x, tx = lin - ty * g.tiles_x;

@@ -20,6 +20,7 @@
 // at (x, x+e1, x+e2) and (z+1).  R3 of the plane below stays in a register.
 #include "solvers.hpp"
 #include "fgp_kernels.hpp"
+#include "deep3d.hpp"
 
 namespace cilreg {
 
@@ -69,7 +70,9 @@ static void launch_fgp2(const Fgp2Args<T, S>& a, bool iso, bool small, hipStream
 // residual (FGP_TV_core.c:66,123).  Iterations run two per pass
 // (fgp2_iter_kernel) unless opts.depth == 1 or, by default, a 2D image has
 // kFgp2dPassMaxPixels or more; an odd last iteration runs on the
-// one-iteration kernel.  2D images in FP32 arithmetic take fgp_solve_2d.  P_j lives in buffer
+// one-iteration kernel.  2D images in FP32 arithmetic take fgp_solve_2d, volumes
+// deep3_fits accepts fgp_solve_3d (not under a scratch limit, whose workspace is
+// this path's).  P_j lives in buffer
 // j mod nbuf (nbuf = 4 with two-iteration passes, which write P_{k+1} and
 // P_{k+2} while reading P_k and P_{k-1}; 3 otherwise).
 template <typename T, typename S>
@@ -84,6 +87,9 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
         // under a scratch limit large images keep the path whose workspace decides what fits
         if (dim == 2 && opts.depth != 1 && !(opts.scratch && (size_t)nx * ny >= kFgp2dPassMaxPixels))
             return fgp_solve_2d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, opts, s, iters_done, re, ws);
+        if (dim == 3 && opts.depth != 1 && !opts.scratch && deep3_fits(nx, ny, nz))
+            return fgp_solve_3d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, opts, s, iters_done, re,
+                                   ws);
     }
     const size_t n = (size_t)nx * ny * nz;
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T) > sizeof(S) ? sizeof(T) : sizeof(S));

@@ -178,21 +178,8 @@ int fgp_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float e
     m.step = 1.0f / (8.0f * lambda);
     m.nonneg = nonneg != 0;
     m.iso = method == 0;
-    // t_k in float (FGP_TV_core.c:138,159); mult[k] multiplies P_k - P_{k-1}
-    std::vector<float> tks(iter + 1);
-    m.mult.resize(iter + 1);
-    float tk = 1, mk = 0;
-    if (ws && ws->warm) {
-        tk = ws->tstate[0];
-        mk = ws->tstate[1];
-    }
-    for (int k = 0; k <= iter; ++k) {
-        m.mult[k] = mk;
-        tks[k] = tk;
-        const float tkp1 = (1.0f + dsqrt_host(1.0f + 4.0f * tk * tk)) * 0.5f;
-        mk = (tk - 1.0f) / tkp1;
-        tk = tkp1;
-    }
+    std::vector<float> tks;
+    fgp_multipliers(iter, ws, m.mult, tks);
     int last = 0;
     if (deep_solve(m, d_f, d_out, nx, ny, iter, epsil, opts, s, iters_done, re, ws, &last) != 0) return -1;
     if (ws) {

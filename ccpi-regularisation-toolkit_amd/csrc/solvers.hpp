@@ -39,11 +39,33 @@ template <typename T>
 int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsil, T eta, int method, int nonneg,
               int nx, int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re);
 
+// FGP's t_k sequence in float (FGP_TV_core.c:138,159), resumed from a warm
+// state: mult[k] multiplies P_k - P_{k-1} in iteration k, tks[k] is t_k.
+inline void fgp_multipliers(int iter, const WarmState* ws, std::vector<float>& mult, std::vector<float>& tks) {
+    mult.resize(iter + 1);
+    tks.resize(iter + 1);
+    float tk = 1, m = 0;
+    if (ws && ws->warm) {
+        tk = ws->tstate[0];
+        m = ws->tstate[1];
+    }
+    for (int k = 0; k <= iter; ++k) {
+        mult[k] = m;
+        tks[k] = tk;
+        const float tkp1 = (1.0f + dsqrt_host(1.0f + 4.0f * tk * tk)) * 0.5f;
+        m = (tk - 1.0f) / tkp1;
+        tk = tkp1;
+    }
+}
+
 // 2D solves with many iterations per launch (opts.depth: 0 = as many as pay,
 // 2 = two; S: storage of the dual fields).
 template <typename S>
 int fgp_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float epsil, int method, int nonneg, int nx,
                  int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws);
+template <typename S>
+int fgp_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float epsil, int method, int nonneg, int nx,
+                 int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws);
 template <typename S>
 int pd_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float epsil, float lipschitz, int method,
                 int nonneg, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re,
