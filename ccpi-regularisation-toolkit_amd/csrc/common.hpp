@@ -372,17 +372,18 @@ template <> struct Mixed<float> {
         if (__builtin_amdgcn_ballot_w64(!(lo == hi))) r = (float)((double)num / c);
         return r;
     }
-    // N quotients with c = 1 + lt and rc = RN(1 / c) at hand: one test for the
-    // wave that divides.
+    // N quotients by c = 1 + lt, rlo / rhi = RN(1 / c) (1 -+ 2^-50) at hand: both
+    // ends are products (they bracket the double quotient as q -+ d do), and
+    // there is one test for the wave that divides.
     template <int N>
-    __device__ static inline void pd_div_n(float (&v)[N], double c, double rc) {
+    __device__ static inline void pd_div_n(float (&v)[N], double c, double rlo, double rhi) {
         float lo[N];
         bool odd = false;
         #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const double q = (double)v[i] * rc, d = fabs(q) * 0x1p-50;
-            lo[i] = (float)(q - d);
-            odd = odd || !(lo[i] == (float)(q + d));
+            const double w = (double)v[i];
+            lo[i] = (float)(w * rlo);
+            odd = odd || !(lo[i] == (float)(w * rhi));
         }
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0, 0)) {
             #pragma unroll

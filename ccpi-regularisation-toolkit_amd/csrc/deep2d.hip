@@ -34,7 +34,7 @@ DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[
 // planes it repeats at the chunk's ends, one step per plane.
 Deep3Plan plan_deep3(int nx, int ny, int nz, int rlo, int rhi, const Deep3Cost (&cost)[kDeep3Shapes], size_t bytes,
                      int most, int zchunk) {
-    constexpr double kCacheBytes = 200e6, kLaunchUs = 4.0;
+    constexpr double kCacheBytes = 200e6, kLaunchUs = 4.0, kAloneStep = 0.75;
     const bool stream = (double)bytes * nx * ny * nz > kCacheBytes;
     Deep3Plan best{};
     double best_us = 1e300;
@@ -49,7 +49,10 @@ Deep3Plan plan_deep3(int nx, int ny, int nz, int rlo, int rhi, const Deep3Cost (
             for (int c = 1; c <= nz; ++c) {
                 const int zc = zchunk > 0 ? zchunk : (nz + c - 1) / c;
                 const int n = (nz + zc - 1) / zc;
-                const double rounds = (double)((regions * n + sh.slots - 1) / sh.slots);
+                // a last round of half the workgroups that fit steps faster
+                const long long rem = regions * n % sh.slots;
+                const double rounds = (double)(regions * n / sh.slots) +
+                                      (rem == 0 ? 0.0 : rem <= sh.slots - 256 ? kAloneStep : 1.0);
                 const double us = (kLaunchUs + rounds * step * (zc + (n > 1 ? lo + hi : t))) / t;
                 if (us < best_us * (1 - 1e-9)) {
                     best_us = us;

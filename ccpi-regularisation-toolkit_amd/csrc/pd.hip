@@ -20,6 +20,7 @@
 // z-1 from a register.
 #include "solvers.hpp"
 #include "pd_kernels.hpp"
+#include "deep3d.hpp"
 #include <vector>
 
 namespace cilreg {
@@ -62,7 +63,8 @@ static void launch_pd2(const Pd2Args<T, S>& a, bool iso, bool small, hipStream_t
     }
 }
 
-// Device-resident PD solve.  In 3D, iterations run two per pass
+// Device-resident PD solve.  Images and (deep3_fits) volumes in FP32 arithmetic
+// take pd_solve_2d and pd_solve_3d; else, in 3D, iterations run two per pass
 // (pd2_iter_kernel) unless opts.depth == 1; an odd last iteration, and every
 // 2D iteration, runs on the one-iteration kernel.  Each pass reads state set
 // `cur` (u_bar, P) and writes set cur ^ 1.  A stop returns the un-extrapolated
@@ -86,6 +88,9 @@ int pd_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, T lipschitz, i
         if (dim == 2 && opts.depth != 1 && nx > 1 && ny > 1)
             return pd_solve_2d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, opts, s, iters_done,
                                   re, ws);
+        if (dim == 3 && opts.depth != 1 && nx > 1 && ny > 1 && deep3_fits(nx, ny, nz))
+            return pd_solve_3d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, nz, opts, s,
+                                  iters_done, re, ws);
     }
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T) > sizeof(S) ? sizeof(T) : sizeof(S));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;

@@ -9,7 +9,7 @@ namespace {
 
 struct PdPar {
     float sigma, tau, lt;
-    double c, rc;        // 1 + lt and its reciprocal
+    double c, rlo, rhi;  // 1 + lt, bounds of its reciprocal
     int nonneg, plain;   // plain: the result is U before extrapolation (a stop), else u_bar
 };
 // state: u_bar, P (2 components)
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(64 * Sh::NW) void pd_deep_kernel(PdDeepArgs a) {
             const T dv = -(q1[r] - deep_left0(p, q1[r])) + -(q2[r] - (r > 0 ? q2[r > 0 ? r - 1 : 0] : above));
             un[r] = u[r] - tau * dv + lt * f[r];
         }
-        Mixed<T>::pd_div_n(un, a.par.c, a.par.rc);
+        Mixed<T>::pd_div_n(un, a.par.c, a.par.rlo, a.par.rhi);
         if ((a.check >> it) & 1u) {
             double sd = 0.0, su = 0.0;
             #pragma unroll
@@ -155,7 +155,8 @@ int pd_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float ep
     m.par.sigma = (float)(1.0 / (double)(lipschitz * m.par.tau));
     m.par.lt = m.par.tau / lambda;
     m.par.c = 1.0 + (double)m.par.lt;
-    m.par.rc = 1.0 / m.par.c;
+    m.par.rlo = 1.0 / m.par.c * (1.0 - 0x1p-50);
+    m.par.rhi = 1.0 / m.par.c * (1.0 + 0x1p-50);
     m.par.nonneg = nonneg != 0;
     m.par.plain = 0;
     m.iso = method == 0;

@@ -67,6 +67,10 @@ template <typename S>
 int fgp_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float epsil, int method, int nonneg, int nx,
                  int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws);
 template <typename S>
+int pd_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float epsil, float lipschitz, int method,
+                int nonneg, int nx, int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re,
+                const WarmState* ws);
+template <typename S>
 int pd_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float epsil, float lipschitz, int method,
                 int nonneg, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re,
                 const WarmState* ws);

@@ -12,12 +12,14 @@ pytestmark = pytest.mark.gpu
 # at least half a million voxels each: smaller volumes take other kernels
 SHAPES = [(2, 520, 500), (3, 411, 409), (600, 29, 31), (520, 1, 1000), (500, 1010, 1), (90, 64, 90), (61, 97, 130),
           (33, 126, 129), (130, 65, 63)]
-METHODS = ["fgp"]
-STORED = {"fgp": ["bf16", "fp16"]}
+METHODS = ["fgp", "pd"]
+STORED = {"fgp": ["bf16", "fp16"], "pd": ["bf16", "fp16"]}
 
 
 def _run(m, x, iters, tol=0.0, nonneg=1, aniso=0, **kw):
     from ccpi.filters import device as D
+    if m == "pd":
+        return D.pd(x, 0.03, iters, tol, 8, aniso, nonneg, **kw)
     return D.fgp(x, 0.03, iters, tol, aniso, nonneg, **kw)
 
 
@@ -104,9 +106,15 @@ def test_warm_start_across_passes(method):
     for kw in ({}, {"tol": 2e-3, "check_every": 1}):
         outs = []
         for depth in (1, 0):
-            st, ts = D.new_state("fgp", x)
-            D.fgp_warm(x, 0.03, 7, st, ts, False, depth=depth, **kw)
-            outs.append((D.fgp_warm(x, 0.03, 14, st, ts, True, depth=depth, **kw), st.clone(), ts.copy()))
+            st = D.new_state(method, x)
+            st, ts = st if method == "fgp" else (st, None)
+            if method == "pd":
+                D.pd_warm(x, 0.03, 7, st, False, depth=depth, **kw)
+                r = D.pd_warm(x, 0.03, 14, st, True, depth=depth, **kw)
+            else:
+                D.fgp_warm(x, 0.03, 7, st, ts, False, depth=depth, **kw)
+                r = D.fgp_warm(x, 0.03, 14, st, ts, True, depth=depth, **kw)
+            outs.append((r, st.clone(), None if ts is None else ts.copy()))
         _same(outs[0][0], outs[1][0], f"{method} {kw}")
         assert bool((outs[0][1] == outs[1][1]).all()), f"{method} {kw}: state"
-        assert np.array_equal(outs[0][2], outs[1][2])
+        assert outs[0][2] is None or np.array_equal(outs[0][2], outs[1][2])
