@@ -34,8 +34,8 @@ DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[
 // planes it repeats at the chunk's ends, one step per plane.
 Deep3Plan plan_deep3(int nx, int ny, int nz, int rlo, int rhi, const Deep3Cost (&cost)[kDeep3Shapes], size_t bytes,
                      int most, int zchunk) {
-    constexpr double kCacheBytes = 200e6, kLaunchUs = 4.0, kAloneStep = 0.75;
-    const bool stream = (double)bytes * nx * ny * nz > kCacheBytes;
+    constexpr double kLaunchUs = 4.0, kAloneStep = 0.75;
+    const bool stream = bytes * nx * ny * nz > kDeep3CacheBytes;
     Deep3Plan best{};
     double best_us = 1e300;
     for (int s = 0; s < kDeep3Shapes; ++s) {

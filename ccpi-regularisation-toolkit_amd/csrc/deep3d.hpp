@@ -12,6 +12,7 @@
 // and repeats T planes at either end of its chunk.
 #pragma once
 #include "deep2d.hpp"
+#include <algorithm>
 
 namespace cilreg {
 
@@ -37,6 +38,9 @@ inline Deep3D make_deep3(int nx, int ny, int nz, int lx, int h, int lo, int hi, 
 // pass then meets the same channels in all of them (256^3 FGP, two iterations
 // per pass: 154 -> 135 us per iteration).
 constexpr size_t kFieldSkew = 17 * 256;
+
+// State that stays in the last-level cache (256 MB) from pass to pass.
+constexpr size_t kDeep3CacheBytes = 200000000;
 
 // The shapes a pass is built in, and how many of its workgroups run at once.
 struct Deep3Shape { int nw, r, slots; };
@@ -157,13 +161,14 @@ struct Deep3Args {
 // deep_solve for volumes: the same state sets, stops, warm starts and output
 // rule.  M supplies Args, NF, rlo, rhi, max (iterations per pass), seeded,
 // field_size, load, store and prepare as there, cost(), bytes() (state per
-// voxel) and launch(T, shape, args, stream).
+// voxel), most(checked) (iterations per pass of a checked or unchecked solve)
+// and launch(T, shape, args, stream).
 template <class M>
 int deep3_solve(M& m, const float* d_f, float* d_out, int nx, int ny, int nz, int iter, float epsil, const Opts& opts,
                 hipStream_t s, int* iters_done, float* re, const WarmState* ws, int* last_iter = nullptr) {
     const size_t n = (size_t)nx * ny * nz;
     const bool use_tol = epsil != 0.0f;
-    const int most = iter < M::max ? iter : M::max;
+    const int most = std::min(iter, m.most(use_tol));
     // shorter passes (the last one, a rerun up to a stop) run on the same regions and chunks
     const Deep3Plan plan = plan_deep3(nx, ny, nz, M::rlo, M::rhi, m.cost(), m.bytes(), most, opts.zchunk);
     const int width = plan.T;

@@ -29,6 +29,7 @@
 // plane below and B of the own point stay in registers.
 #include "solvers.hpp"
 #include "fgp_kernels.hpp"
+#include "deep3d.hpp"
 
 namespace cilreg {
 
@@ -607,7 +608,8 @@ static void launch_dtv(const DtvArgs<T>& a, bool iso, bool small, hipStream_t s)
     }
 }
 
-// Device-resident FGP-dTV solve.  d_out receives D of the final iteration
+// Device-resident FGP-dTV solve; volumes that deep3_fits accepts run on
+// dtv_solve_3d unless opts.depth == 1.  d_out receives D of the final iteration
 // (left untouched when iter == 0); with epsil != 0 its prior contents seed the
 // first residual (FGP_dTV_core.c:78,131).
 template <typename T>
@@ -619,6 +621,46 @@ int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsi
     *re = 0.f;
     if (iter <= 0) return 0;
     const size_t n = (size_t)nx * ny * nz;
+    // t_k with a double square root and a double sum rounded once
+    // (FGP_dTV_core.c:95,149); mult[k] multiplies (P_k - P_{k-1}) in iteration k
+    std::vector<T> mult(iter + 1);
+    {
+        T tk = 1, m = 0;
+        for (int k = 0; k <= iter; ++k) {
+            mult[k] = m;
+            const T tkp1 = (T)((1.0 + sqrt((double)((T)1 + (T)4 * tk * tk))) * 0.5);
+            m = (tk - (T)1) / tkp1;
+            tk = tkp1;
+        }
+    }
+    // B on the solve's stream
+    auto refgrad = [&](T* const (&B)[3]) {
+        size_t blocks = (n + 255) / 256;
+        if (blocks > 65536) blocks = 65536;
+        if (dim == 3)
+            hipLaunchKernelGGL((dtv_refgrad_kernel<3, T>), dim3((unsigned)blocks), dim3(256), 0, s, d_ref, B[0], B[1],
+                               B[2], eta, nx, ny, nz);
+        else
+            hipLaunchKernelGGL((dtv_refgrad_kernel<2, T>), dim3((unsigned)blocks), dim3(256), 0, s, d_ref, B[0], B[1],
+                               B[2], eta, nx, ny, nz);
+    };
+    if constexpr (std::is_same<T, float>::value) {
+        // Checked passes have two levels (three spill), which pay unless the
+        // fields stream from HBM in rows of whole 128-byte lines, the tiled
+        // pass's best case: 256^3 checked every fifth iteration 157 us tiled and
+        // 176 in registers, 190 x 257 x 231 163 and 105, 128^3 25.6 and 22.2.
+        const bool tiled = epsil != (T)0 && nx % 32 == 0 && n * 64 > kDeep3CacheBytes;
+        if (dim == 3 && opts.depth != 1 && deep3_fits(nx, ny, nz) && !tiled) {
+            Arena ar;
+            size_t oB[3];
+            for (size_t& o : oB) o = ar.reserve(n * sizeof(float) + kFieldSkew);
+            if (ar.allocate() != 0) return -1;
+            float* const B[3] = {(float*)ar.at(oB[0]), (float*)ar.at(oB[1]), (float*)ar.at(oB[2])};
+            refgrad(B);
+            return dtv_solve_3d(d_f, {B[0], B[1], B[2]}, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, mult,
+                                opts, s, iters_done, re);
+        }
+    }
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;
     const bool iso = method == 0;
@@ -656,16 +698,7 @@ int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsi
     auto Pbuf = [&](int j, int c) -> T* { return (T*)ar.at(oP[((j % nbuf) + nbuf) % nbuf][c < dim ? c : 0]); };
     T* B[3];
     for (int c = 0; c < 3; ++c) B[c] = (T*)ar.at(oB[c < dim ? c : 0]);
-    {
-        size_t blocks = (n + 255) / 256;
-        if (blocks > 65536) blocks = 65536;
-        if (dim == 3)
-            hipLaunchKernelGGL((dtv_refgrad_kernel<3, T>), dim3((unsigned)blocks), dim3(256), 0, s, d_ref, B[0], B[1],
-                               B[2], eta, nx, ny, nz);
-        else
-            hipLaunchKernelGGL((dtv_refgrad_kernel<2, T>), dim3((unsigned)blocks), dim3(256), 0, s, d_ref, B[0], B[1],
-                               B[2], eta, nx, ny, nz);
-    }
+    refgrad(B);
     const bool use_tol = epsil != (T)0;
     T* Dbuf[2] = {(T*)ar.at(oD[0]), (T*)ar.at(oD[1])};
     if (use_tol) launch_copy(Dbuf[1], d_out, n * sizeof(T), s);   // D_{-1} = caller's Output
@@ -676,18 +709,6 @@ int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsi
     auto needs_d = [&](int k) { return k == iter - 1 || (use_tol && (k % ce == 0 || (k + 1) % ce == 0)); };
     const T stepc = (T)1 / ((dim == 3 ? (T)26 : (T)8) * lambda);
 
-    // t_k with a double square root and a double sum rounded once
-    // (FGP_dTV_core.c:95,149); mult[k] multiplies (P_k - P_{k-1}) in iteration k
-    std::vector<T> mult(iter + 1);
-    {
-        T tk = 1, m = 0;
-        for (int k = 0; k <= iter; ++k) {
-            mult[k] = m;
-            const T tkp1 = (T)((1.0 + sqrt((double)((T)1 + (T)4 * tk * tk))) * 0.5);
-            m = (tk - (T)1) / tkp1;
-            tk = tkp1;
-        }
-    }
     // one iteration k on the one-iteration kernel
     auto one = [&](int k, bool write_d, bool check, const Ctrl* c_ptr) {
         DtvArgs<T> a;

@@ -81,147 +81,142 @@ __global__ __launch_bounds__(64 * Sh::NW, 4) void pd_deep3_kernel(Pd3Args a) {
         #pragma unroll
         for (int c = 0; c < 3; ++c) landed(lp[r][c]);
     }
-    // one plane of every level; parity: the step's
-    auto march = [&](int zi, auto parity) {
-        const int b = parity;
-        float iu[R], ip[R][3], fi[R];   // the level's input at its plane: u_bar, P, f
+    // one plane of every level per step, two steps per turn: what one carries on
+    // lands in registers that the other has freed (T = 3 on 8 waves 4-6% faster;
+    // deeper and checked passes would spill)
+    constexpr int U = !CHK && T < 4 ? 2 : 1;
+    for (int zu = zs, parity = 0; zu <= ze; zu += U, parity ^= U & 1) {
         #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            iu[r] = lu[r];
-            fi[r] = lf[r];
-            #pragma unroll
-            for (int c = 0; c < 3; ++c) ip[r][c] = PlaneIn<S>::value(lp[r][c]);
-        }
-        load(zi + 1);
-        #pragma unroll
-        for (int i = 0; i < T; ++i) {
-            const int zc = zi - i, zp = zc - 1, ex = (i + b * T) & 1;
-            rowU[i][b][0][p.grp][p.lx] = iu[0];
-            rowU[i][b][1][p.grp][p.lx] = iu[R - 1];
-            // the dual step at plane zp
-            const float ubl = rowU[i][b ^ 1][0][p.grp + 1 < G ? p.grp + 1 : p.grp][p.lx];
-            float q1[R], q2[R], q3[R], ux[R], uy[R], uz[R];
+        for (int h = 0; h < U; ++h) {
+            const int zi = zu + h, b = U == 2 ? h : parity;
+            if (h > 0 && zi > ze) break;
+            float iu[R], ip[R][3], fi[R];   // the level's input at its plane: u_bar, P, f
             #pragma unroll
             for (int r = 0; r < R; ++r) {
-                ux[r] = deep_right(cu[i][r]);
-                uy[r] = r + 1 < R ? cu[i][r + 1 < R ? r + 1 : r] : ubl;
-                uz[r] = iu[r];
+                iu[r] = lu[r];
+                fi[r] = lf[r];
+                #pragma unroll
+                for (int c = 0; c < 3; ++c) ip[r][c] = PlaneIn<S>::value(lp[r][c]);
             }
-            if (p.xedge) {
-                deep_keep_branch();
+            load(zi + 1);
+            #pragma unroll
+            for (int i = 0; i < T; ++i) {
+                const int zc = zi - i, zp = zc - 1, ex = (i + b * T) & 1;
+                rowU[i][b][0][p.grp][p.lx] = iu[0];
+                rowU[i][b][1][p.grp][p.lx] = iu[R - 1];
+                // the dual step at plane zp
+                const float ubl = rowU[i][b ^ 1][0][p.grp + 1 < G ? p.grp + 1 : p.grp][p.lx];
+                float q1[R], q2[R], q3[R], ux[R], uy[R], uz[R];
                 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    const float l = deep_left(cu[i][r]);
-                    ux[r] = xlast ? l : ux[r];
+                    ux[r] = deep_right(cu[i][r]);
+                    uy[r] = r + 1 < R ? cu[i][r + 1 < R ? r + 1 : r] : ubl;
+                    uz[r] = iu[r];
                 }
-            }
-            if (p.yedge) {
-                deep_keep_branch();
-                const float uab = rowU[i][b ^ 1][1][p.grp > 0 ? p.grp - 1 : 0][p.lx];
-                #pragma unroll
-                for (int r = 0; r < R; ++r)
-                    uy[r] = p.y + r == p.ny - 1 ? (r > 0 ? cu[i][r > 0 ? r - 1 : 0] : uab) : uy[r];
-            }
-            if (zp == nz - 1) {
-                deep_keep_branch();
-                #pragma unroll
-                for (int r = 0; r < R; ++r) uz[r] = bu[i][r];
-            }
-            #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                q1[r] = cp[i][r][0] + sigma * (ux[r] - cu[i][r]);
-                q2[r] = cp[i][r][1] + sigma * (uy[r] - cu[i][r]);
-                q3[r] = cp[i][r][2] + sigma * (uz[r] - cu[i][r]);
-            }
-            project_unit_n<3, float, ISO>(q1, q2, q3);
-            rowQ[ex][p.grp][p.lx] = q2[R - 1];
-            __syncthreads();
-            const float qab = rowQ[ex][p.grp > 0 ? p.grp - 1 : 0][p.lx];
-            const float above = p.grp > 0 ? qab : 0.0f;   // P2(-1) = 0 at the first row
-            if (zp == 0) {
-                deep_keep_branch();
-                #pragma unroll
-                for (int r = 0; r < R; ++r) bq[i][r] = 0.0f;   // P3(-1) = 0
-            }
-            // the primal step at plane zp; -(q - 0) is -q
-            float u0[R], un[R];
-            #pragma unroll
-            for (int r = 0; r < R; ++r) u0[r] = cu[i][r];
-            if (nonneg) {
-                #pragma unroll
-                for (int r = 0; r < R; ++r) u0[r] = u0[r] < 0.0f ? 0.0f : u0[r];
-            }
-            #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float v1 = -(q1[r] - deep_left(q1[r])), v2 = -(q2[r] - (r > 0 ? q2[r > 0 ? r - 1 : 0] : above));
-                const float v3 = -(q3[r] - bq[i][r]);
-                const float dv = v1 + v2 + v3;
-                un[r] = u0[r] - tau * dv + lt * cf[i][r];
-            }
-            Mixed<float>::pd_div_n(un, a.par.c, a.par.rlo, a.par.rhi);
-            const bool inz = zp >= z0 && zp < z1;
-            if (CHK && inz && ((a.check >> i) & 1u)) {
-                double sd = 0.0, su = 0.0;
-                #pragma unroll
-                for (int r = 0; r < R; ++r)
-                    if (p.out(r)) {
-                        const float df = un[r] - u0[r];
-                        sd += (double)df * (double)df;
-                        su += (double)un[r] * (double)un[r];
-                    }
-                acc[2 * i][tid] += sd;
-                acc[2 * i + 1][tid] += su;
-            }
-            if (i == T - 1) {
-                const size_t zo = plane_offset(zp, p.sxy);
-                const PlaneOut<float> pr(a.res + zo, inz && a.write_res, p.sxy);
-                const PlaneOut<float> pu((float*)a.out[0] + zo, inz && a.write_state, p.sxy);
-                #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const float v = un[r] + (un[r] - u0[r]);
-                    pu.st(so[r], v);
-                    pr.st(so[r], a.par.plain ? un[r] : v);
-                }
-                #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const PlaneOut<S> pp((S*)a.out[1 + c] + zo, inz && a.write_state, p.sxy);
+                if (p.xedge) {
+                    deep_keep_branch();
                     #pragma unroll
-                    for (int r = 0; r < R; ++r) pp.st(so[r], c == 0 ? q1[r] : c == 1 ? q2[r] : q3[r]);
+                    for (int r = 0; r < R; ++r) {
+                        const float l = deep_left(cu[i][r]);
+                        ux[r] = xlast ? l : ux[r];
+                    }
+                }
+                if (p.yedge) {
+                    deep_keep_branch();
+                    const float uab = rowU[i][b ^ 1][1][p.grp > 0 ? p.grp - 1 : 0][p.lx];
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        uy[r] = p.y + r == p.ny - 1 ? (r > 0 ? cu[i][r > 0 ? r - 1 : 0] : uab) : uy[r];
+                }
+                if (zp == nz - 1) {
+                    deep_keep_branch();
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r) uz[r] = bu[i][r];
+                }
+                #pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    q1[r] = cp[i][r][0] + sigma * (ux[r] - cu[i][r]);
+                    q2[r] = cp[i][r][1] + sigma * (uy[r] - cu[i][r]);
+                    q3[r] = cp[i][r][2] + sigma * (uz[r] - cu[i][r]);
+                }
+                project_unit_n<3, float, ISO>(q1, q2, q3);
+                rowQ[ex][p.grp][p.lx] = q2[R - 1];
+                __syncthreads();
+                const float qab = rowQ[ex][p.grp > 0 ? p.grp - 1 : 0][p.lx];
+                const float above = p.grp > 0 ? qab : 0.0f;   // P2(-1) = 0 at the first row
+                if (zp == 0) {
+                    deep_keep_branch();
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r) bq[i][r] = 0.0f;   // P3(-1) = 0
+                }
+                // the primal step at plane zp; -(q - 0) is -q
+                float u0[R], un[R];
+                #pragma unroll
+                for (int r = 0; r < R; ++r) u0[r] = cu[i][r];
+                if (nonneg) {
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r) u0[r] = u0[r] < 0.0f ? 0.0f : u0[r];
+                }
+                #pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float v1 = -(q1[r] - deep_left(q1[r])), v2 = -(q2[r] - (r > 0 ? q2[r > 0 ? r - 1 : 0] : above));
+                    const float v3 = -(q3[r] - bq[i][r]);
+                    const float dv = v1 + v2 + v3;
+                    un[r] = u0[r] - tau * dv + lt * cf[i][r];
+                }
+                Mixed<float>::pd_div_n(un, a.par.c, a.par.rlo, a.par.rhi);
+                const bool inz = zp >= z0 && zp < z1;
+                if (CHK && inz && ((a.check >> i) & 1u)) {
+                    double sd = 0.0, su = 0.0;
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (p.out(r)) {
+                            const float df = un[r] - u0[r];
+                            sd += (double)df * (double)df;
+                            su += (double)un[r] * (double)un[r];
+                        }
+                    acc[2 * i][tid] += sd;
+                    acc[2 * i + 1][tid] += su;
+                }
+                if (i == T - 1) {
+                    const size_t zo = plane_offset(zp, p.sxy);
+                    const PlaneOut<float> pr(a.res + zo, inz && a.write_res, p.sxy);
+                    const PlaneOut<float> pu((float*)a.out[0] + zo, inz && a.write_state, p.sxy);
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float v = un[r] + (un[r] - u0[r]);
+                        pu.st(so[r], v);
+                        pr.st(so[r], a.par.plain ? un[r] : v);
+                    }
+                    #pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const PlaneOut<S> pp((S*)a.out[1 + c] + zo, inz && a.write_state, p.sxy);
+                        #pragma unroll
+                        for (int r = 0; r < R; ++r) pp.st(so[r], c == 0 ? q1[r] : c == 1 ? q2[r] : q3[r]);
+                    }
+                }
+                if (zc == nz - 1) {   // the last plane's forward difference reads the plane below it
+                    deep_keep_branch();
+                    #pragma unroll
+                    for (int r = 0; r < R; ++r) bu[i][r] = cu[i][r];
+                }
+                // carry this plane; the next level takes u_bar, P and f of plane zp
+                #pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float of = cf[i][r];
+                    bq[i][r] = q3[r];
+                    cu[i][r] = iu[r];
+                    cf[i][r] = fi[r];
+                    #pragma unroll
+                    for (int c = 0; c < 3; ++c) cp[i][r][c] = ip[r][c];
+                    iu[r] = un[r] + (un[r] - u0[r]);
+                    ip[r][0] = through_storage<float, S>(q1[r]);
+                    ip[r][1] = through_storage<float, S>(q2[r]);
+                    ip[r][2] = through_storage<float, S>(q3[r]);
+                    fi[r] = of;
                 }
             }
-            if (zc == nz - 1) {   // the last plane's forward difference reads the plane below it
-                deep_keep_branch();
-                #pragma unroll
-                for (int r = 0; r < R; ++r) bu[i][r] = cu[i][r];
-            }
-            // carry this plane; the next level takes u_bar, P and f of plane zp
-            #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float of = cf[i][r];
-                bq[i][r] = q3[r];
-                cu[i][r] = iu[r];
-                cf[i][r] = fi[r];
-                #pragma unroll
-                for (int c = 0; c < 3; ++c) cp[i][r][c] = ip[r][c];
-                iu[r] = un[r] + (un[r] - u0[r]);
-                ip[r][0] = through_storage<float, S>(q1[r]);
-                ip[r][1] = through_storage<float, S>(q2[r]);
-                ip[r][2] = through_storage<float, S>(q3[r]);
-                fi[r] = of;
-            }
         }
-    };
-    if constexpr (T < 4) {
-        // two steps per turn: what one carries on lands in registers that the
-        // other has freed (a third of the moves gone, T = 3 on 8 waves 5%
-        // faster; T = 4 with 16-bit P would spill and gains nothing)
-        for (int zi = zs; zi <= ze; zi += 2) {
-            march(zi, std::integral_constant<int, 0>{});
-            if (zi == ze) break;
-            march(zi + 1, std::integral_constant<int, 1>{});
-        }
-    } else {
-        for (int zi = zs, b = 0; zi <= ze; ++zi, b ^= 1) march(zi, b);
     }
     if (CHK) {
         int n = 0;
@@ -254,6 +249,7 @@ struct Pd3 {
     static constexpr bool seeded = false;
     Pd3Par par;
     bool iso;
+    int most(bool) const { return max; }
     size_t field_size(int i) const { return i == 0 ? sizeof(float) : sizeof(S); }
     const Deep3Cost (&cost() const)[kDeep3Shapes] { return sizeof(S) == 4 ? kPd3Cost : kPd3Cost16; }
     size_t bytes() const { return 6 * sizeof(S) + 12; }

@@ -66,6 +66,9 @@ int fgp_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float e
 template <typename S>
 int fgp_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float epsil, int method, int nonneg, int nx,
                  int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws);
+int dtv_solve_3d(const float* d_f, const float* const (&B)[3], float* d_out, float lambda, int iter, float epsil,
+                 int method, int nonneg, int nx, int ny, int nz, const std::vector<float>& mult, const Opts& opts,
+                 hipStream_t s, int* iters_done, float* re);
 template <typename S>
 int pd_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float epsil, float lipschitz, int method,
                 int nonneg, int nx, int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re,

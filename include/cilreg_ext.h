@@ -43,8 +43,8 @@ typedef struct cilreg_opts {
     int profile;         /* 1: time every iteration's kernels with HIP events (see cilreg_last_profile) */
     int wide_index;      /* 1: force 64-bit element indexing (chosen automatically for fields >= 2 GiB) */
     int stream_launches; /* batch: 1 = launch directly instead of capturing one hipGraph */
-    int temporal_depth;  /* iterations fused per pass where supported: 0 = auto (3D FGP, PD: up to 4, TGV: 2;
-                            2D: up to 8), 1 = off, 2 = two (3D FGP, PD: as 0) */
+    int temporal_depth;  /* iterations fused per pass where supported: 0 = auto (3D FGP, PD: up to 4, dTV: 3, TGV: 2;
+                            2D: up to 8), 1 = off, 2 = two (3D FGP, PD, dTV: as 0) */
     int autotune;        /* 1: tile_y / zchunk / temporal_depth left at 0 are chosen by cilreg_autotune */
     int persistent;      /* batch: 1 = one persistent work-queue kernel per method group; disabled in this
                             build (cilreg_batch_run returns -1 with the reason) */

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 # at least half a million voxels each: smaller volumes take other kernels
 SHAPES = [(2, 520, 500), (3, 411, 409), (600, 29, 31), (520, 1, 1000), (500, 1010, 1), (90, 64, 90), (61, 97, 130),
           (33, 126, 129), (130, 65, 63)]
-METHODS = ["fgp", "pd"]
+METHODS = ["fgp", "pd", "dtv"]
 STORED = {"fgp": ["bf16", "fp16"], "pd": ["bf16", "fp16"]}
 
 
@@ -20,6 +20,8 @@ def _run(m, x, iters, tol=0.0, nonneg=1, aniso=0, **kw):
     from ccpi.filters import device as D
     if m == "pd":
         return D.pd(x, 0.03, iters, tol, 8, aniso, nonneg, **kw)
+    if m == "dtv":
+        return D.dtv(x, _vol(tuple(x.shape), 99), 0.03, iters, tol, 0.05, aniso, nonneg, **kw)
     return D.fgp(x, 0.03, iters, tol, aniso, nonneg, **kw)
 
 
@@ -53,7 +55,7 @@ def test_equal_to_one_iteration_per_launch(method, shape):
     _same(_run(method, x, 7, depth=1), _run(method, x, 7, depth=2), f"{method} {shape} depth 2")
 
 
-@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("method", ["fgp", "pd"])
 def test_16bit_storage(method):
     x = _vol((70, 90, 100), 4)
     for precision in STORED[method]:
@@ -99,7 +101,7 @@ def test_values_outside_the_fast_ranges(method):
         _same(_run(method, y, 7, nonneg=0, depth=1), _run(method, y, 7, nonneg=0), f"{method} {bad}")
 
 
-@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("method", ["fgp", "pd"])
 def test_warm_start_across_passes(method):
     from ccpi.filters import device as D
     x = _vol((60, 91, 97), 8)
