@@ -25,6 +25,11 @@
 // The work per voxel is arithmetic (divisions and square roots on every
 // flux), so these kernels are bounded by the vector ALUs rather than HBM.
 //
+// LLT-ROF measured in 3D (before: IEEE division and square roots, every plane's
+// z neighbours loaded again, ring lanes through both branches): 256^3 119 -> 101
+// us per iteration, 150 x 201 x 180 48.5 -> 41.4, 128^3 19.3 -> 16.2; 12 -> 6
+// loads per point, which gave more than the arithmetic (4%).
+//
 // Fusion: a workgroup owns a 64 x TY column tile and marches through a chunk
 // of z.  For each plane the quantities the update reads at x +- 1 / y +- 1
 // (u for NDF, the LLT and ROF fluxes, W for Diff4th) go through LDS planes of
@@ -286,37 +291,40 @@ __global__ __launch_bounds__(TX * TY) void ndf_iter_kernel(DiffArgs<float> a) {
 // u_dd / (|u_dd| + 1e-12), the denominator rounded from double (LLT_ROF_core.c:145-152)
 __device__ inline float llt_ratio(float dd) { return dd / (float)(fabs((double)dd) + 1.0e-12); }
 
-// ROF fluxes (floor 1e-12) and the x / y second-order terms at a point
+// Two of them: in range (numerators 0 or from 2^-100 up and below 2^60), both
+// by div_in; a wave with any other lane divides.
+__device__ inline void llt_ratio2(float a, float b, float& ra, float& rb) {
+    const float sum = fabsf(a) + fabsf(b);   // NaN if either is
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum < 0x1p+60f) ||
+                                                     min_key(tiny_key(a), tiny_key(b)) < kTinyKey) != 0, 0)) {
+        ra = llt_ratio(a);
+        rb = llt_ratio(b);
+        return;
+    }
+    const float da = (float)(fabs((double)a) + 1.0e-12), db = (float)(fabs((double)b) + 1.0e-12);
+    ra = div_in(a, da, rcp_in(da));
+    rb = div_in(b, db, rcp_in(db));
+}
+
+__device__ inline float llt_ratio1(float a) {
+    float r, unused;
+    llt_ratio2(a, 0.0f, r, unused);
+    return r;
+}
+
+// ROF fluxes (floor 1e-12) and the x / y second-order terms at a point, from u
+// there and at its z neighbours
 template <int DIM, typename I>
-__device__ inline void llt_point(const DiffArgs<float>& a, int px, int py, int z, float& r1, float& r2, float& r3,
-                                 float& l1, float& l2) {
+__device__ inline void llt_point(const DiffArgs<float>& a, int px, int py, int z, float uc, float ukp, float ukm,
+                                 float& r1, float& r2, float& r3, float& l1, float& l2) {
     const Geom& g = a.g;
-    const I sxy = (I)g.sxy, nx = (I)g.nx;
-    const I zo = (I)z * sxy, c = zo + (I)py * nx + (I)px;
-    const float uc = ldx<float>(a.U, c);
+    const I nx = (I)g.nx, zo = (I)z * (I)g.sxy;
     const float uip = ldx<float>(a.U, zo + (I)py * nx + (I)mirror_p(px, g.nx));
     const float uim = ldx<float>(a.U, zo + (I)py * nx + (I)mirror_m(px, g.nx));
     const float ujp = ldx<float>(a.U, zo + (I)mirror_p(py, g.ny) * nx + (I)px);
     const float ujm = ldx<float>(a.U, zo + (I)mirror_m(py, g.ny) * nx + (I)px);
-    float ukp = 0.f, ukm = 0.f;
-    if (DIM == 3) {
-        ukp = ldx<float>(a.U, (I)mirror_p(z, g.nz) * sxy + (I)py * nx + (I)px);
-        ukm = ldx<float>(a.U, (I)mirror_m(z, g.nz) * sxy + (I)py * nx + (I)px);
-    }
     rof_flux_math<DIM, float>(uc, uip, uim, ujp, ujm, ukp, ukm, r1, r2, r3, 1.0e-12);
-    l1 = llt_ratio(uip - 2.0f * uc + uim);
-    l2 = llt_ratio(ujp - 2.0f * uc + ujm);
-}
-
-// the z second-order term of the own column at plane z
-template <typename I>
-__device__ inline float llt_l3(const DiffArgs<float>& a, I col, int z) {
-    const Geom& g = a.g;
-    const I sxy = (I)g.sxy;
-    const float uc = ldx<float>(a.U, (I)z * sxy + col);
-    const float up = ldx<float>(a.U, (I)mirror_p(z, g.nz) * sxy + col);
-    const float um = ldx<float>(a.U, (I)mirror_m(z, g.nz) * sxy + col);
-    return llt_ratio(up - 2.0f * uc + um);
+    llt_ratio2(uip - 2.0f * uc + uim, ujp - 2.0f * uc + ujm, l1, l2);
 }
 
 template <int DIM, int TY, typename I>
@@ -335,19 +343,30 @@ __device__ inline void llt_body(const DiffArgs<float>& a, const TileCoord& tc) {
     const int sxp = own ? mirror_p(x, g.nx) - tc.x0 + 1 : lx + 1, sxm = own ? mirror_m(x, g.nx) - tc.x0 + 1 : lx + 1;
     const int syp = own ? mirror_p(y, g.ny) - tc.y0 + 1 : ly + 1, sym = own ? mirror_m(y, g.ny) - tc.y0 + 1 : ly + 1;
 
+    // u of the own column at mirrored planes: um, uc, up at z - 1, z, z + 1; each
+    // plane loads only z + 2 of it
+    auto ucol = [&](int z) { return ldx<float>(a.U, (I)z * sxy + col); };
+    float uc = ucol(tc.z0), um = 0.f, up = 0.f;
     float r3m = 0.f, l3m = 0.f, l3c = 0.f;   // D_rof,3 and D_llt,3 of the own column below / here
     if (DIM == 3) {
+        const int zm = mirror_m(tc.z0, g.nz);
+        um = ucol(zm);
+        up = ucol(mirror_p(tc.z0, g.nz));
+        const float b = ucol(mirror_m(zm, g.nz)), t = ucol(mirror_p(zm, g.nz));
         float t1, t2, t4, t5;
-        llt_point<DIM, I>(a, ox, oy, mirror_m(tc.z0, g.nz), t1, t2, r3m, t4, t5);
-        l3m = llt_l3<I>(a, col, mirror_m(tc.z0, g.nz));
-        l3c = llt_l3<I>(a, col, tc.z0);
+        llt_point<DIM, I>(a, ox, oy, zm, um, t, b, t1, t2, r3m, t4, t5);
+        l3m = llt_ratio1(t - 2.0f * um + b);
+        l3c = llt_ratio1(up - 2.0f * uc + um);
     }
     double sdd = 0.0, suu = 0.0;
     for (int z = tc.z0; z < tc.z1; ++z) {
+        float upp = 0.f;
+        if (DIM == 3) upp = ucol(mirror_p(z + 1 < g.nz ? z + 1 : z, g.nz));
+        else uc = ucol(z);
         float r1, r2, r3, l1, l2;
-        llt_point<DIM, I>(a, ox, oy, z, r1, r2, r3, l1, l2);
+        llt_point<DIM, I>(a, ox, oy, z, uc, up, um, r1, r2, r3, l1, l2);
         float l3p = 0.f;
-        if (DIM == 3) l3p = (z + 1 < g.nz) ? llt_l3<I>(a, col, z + 1) : l3m;
+        if (DIM == 3) l3p = (z + 1 < g.nz) ? llt_ratio1(upp - 2.0f * up + uc) : l3m;
         L1s[ly + 1][lx + 1] = l1;
         L2s[ly + 1][lx + 1] = l2;
         R1s[ly + 1][lx + 1] = r1;
@@ -355,34 +374,30 @@ __device__ inline void llt_body(const DiffArgs<float>& a, const TileCoord& tc) {
         if (r.lane) {
             // only what the tile reads at the lane's slot: L1 on the columns
             // and D2 on the left one, L2 on the rows and D1 on the upper one
+            // (p / m: the neighbours along that axis, op / om: across it)
             const I zo = (I)z * sxy, rc = zo + (I)r.y * nx + (I)r.x;
-            const float uc = ldx<float>(a.U, rc);
-            const float uip = ldx<float>(a.U, zo + (I)r.y * nx + (I)mirror_p(r.x, g.nx));
-            const float uim = ldx<float>(a.U, zo + (I)r.y * nx + (I)mirror_m(r.x, g.nx));
-            const float ujp = ldx<float>(a.U, zo + (I)mirror_p(r.y, g.ny) * nx + (I)r.x);
-            const float ujm = ldx<float>(a.U, zo + (I)mirror_m(r.y, g.ny) * nx + (I)r.x);
-            float mk = 0.f;
-            if (DIM == 3) {
-                const float ukp = ldx<float>(a.U, (I)mirror_p(z, g.nz) * sxy + (I)r.y * nx + (I)r.x);
-                const float ukm = ldx<float>(a.U, (I)mirror_m(z, g.nz) * sxy + (I)r.y * nx + (I)r.x);
-                mk = Mixed<float>::minmod_sq(ukp - uc, uc - ukm);
+            const bool side = r.sx == 0 || r.sx == TX + 1;
+            const I xp = zo + (I)r.y * nx + (I)mirror_p(r.x, g.nx), xm = zo + (I)r.y * nx + (I)mirror_m(r.x, g.nx);
+            const I yp = zo + (I)mirror_p(r.y, g.ny) * nx + (I)r.x, ym = zo + (I)mirror_m(r.y, g.ny) * nx + (I)r.x;
+            const float hc = ldx<float>(a.U, rc);
+            const float hp = ldx<float>(a.U, side ? xp : yp), hm = ldx<float>(a.U, side ? xm : ym);
+            float* ls = side ? &L1s[r.sy][r.sx] : &L2s[r.sy][r.sx];
+            if (r.sx == 0 || r.sy == 0) {
+                const float uop = ldx<float>(a.U, side ? yp : xp), uom = ldx<float>(a.U, side ? ym : xm);
+                float fk = 0.f, bk = 0.f;
+                if (DIM == 3) {
+                    fk = ldx<float>(a.U, (I)mirror_p(z, g.nz) * sxy + (I)r.y * nx + (I)r.x) - hc;
+                    bk = hc - ldx<float>(a.U, (I)mirror_m(z, g.nz) * sxy + (I)r.y * nx + (I)r.x);
+                }
+                const float q = rof_ring_flux<DIM>(side, hp - hc, uop - hc, hc - uom, fk, bk, 1.0e-12);
+                if (side) R2s[r.sy][r.sx] = q;
+                else R1s[r.sy][r.sx] = q;
             }
-            if (r.sx == 0 || r.sx == TX + 1) {
-                L1s[r.sy][r.sx] = llt_ratio(uip - 2.0f * uc + uim);
-                if (r.sx == 0)
-                    R2s[r.sy][r.sx] = rof_d2<DIM, float>(uip - uc, Mixed<float>::minmod_sq(ujp - uc, uc - ujm), mk,
-                                                          1.0e-12);
-            } else {
-                L2s[r.sy][r.sx] = llt_ratio(ujp - 2.0f * uc + ujm);
-                if (r.sy == 0)
-                    R1s[r.sy][r.sx] = rof_d1<DIM, float>(ujp - uc, Mixed<float>::minmod_sq(uip - uc, uc - uim), mk,
-                                                          1.0e-12);
-            }
+            *ls = llt_ratio1(hp - 2.0f * hc + hm);
         }
         __syncthreads();
         if (own) {
             const I i = (I)z * sxy + col;
-            const float uc = ldx<float>(a.U, i);
             float lap = (L1s[ly + 1][sxp] - 2.0f * l1 + L1s[ly + 1][sxm]) + (L2s[syp][lx + 1] - 2.0f * l2 + L2s[sym][lx + 1]);
             float dv = (r1 - R1s[sym][lx + 1]) + (r2 - R2s[ly + 1][sxm]);
             if (DIM == 3) {
@@ -397,12 +412,20 @@ __device__ inline void llt_body(const DiffArgs<float>& a, const TileCoord& tc) {
         r3m = r3;
         l3m = l3c;
         l3c = l3p;
+        um = uc;
+        uc = up;
+        up = upp;
     }
     if (a.check) store_partials<TY>(a, tc, tid, sdd, suu);
 }
 
+// 64 VGPRs keep four 512-thread workgroups on a CU in 3D (66 without the cap,
+// three workgroups: 256^3 118 -> 131 us per iteration).
+template <int DIM, typename I>
+constexpr int llt_waves() { return DIM == 3 && sizeof(I) == 4 ? 8 : 1; }
 template <int DIM, int TY, typename I>
-__global__ __launch_bounds__(TX * TY) void llt_iter_kernel(DiffArgs<float> a) {
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(llt_waves<DIM, I>())))
+void llt_iter_kernel(DiffArgs<float> a) {
     if (solve_stopped(a.ctrl)) return;
     llt_body<DIM, TY, I>(a, tile_of_block(a.g, TY));
 }

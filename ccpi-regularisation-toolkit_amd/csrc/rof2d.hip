@@ -17,7 +17,7 @@ using RofDeepArgs = DeepArgs<float, 1, RofPar>;   // state: u
 // take sqrt_in and div_in; one test sends a wave with any other point --
 // a difference that is NaN or overflows (the products and squares are summed:
 // any of them makes the sum NaN or infinite), or a numerator below 2^-100 --
-// to rof_flux_math.
+// to rof_flux_ref.
 template <int N>
 __device__ inline void rof2d_fluxes(const float (&uc)[N], const float (&ul)[N], const float (&ur)[N],
                                     const float (&uu)[N], const float (&ud)[N], float (&d1)[N], float (&d2)[N]) {
@@ -42,7 +42,7 @@ __device__ inline void rof2d_fluxes(const float (&uc)[N], const float (&ul)[N], 
         #pragma unroll
         for (int r = 0; r < N; ++r) {
             float d3;
-            rof_flux_math<2, float>(uc[r], ur[r], ul[r], ud[r], uu[r], 0.f, 0.f, d1[r], d2[r], d3);
+            rof_flux_ref<2, float>(uc[r], ur[r], ul[r], ud[r], uu[r], 0.f, 0.f, d1[r], d2[r], d3, 1.0e-8);
         }
         return;
     }

@@ -42,10 +42,11 @@ __device__ inline T rof_d2(T fi, T mj, T mk, double eps) {
 }
 
 // The fluxes D1, D2 and, in 3D, D3 (along z, ROF_TV_core.c:257-263) at a
-// point from u there (uc) and at its mirrored neighbours.
+// point from u there (uc) and at its mirrored neighbours, as the reference
+// writes them.
 template <int DIM, typename T>
-__device__ inline void rof_flux_math(T uc, T uip, T uim, T ujp, T ujm, T ukp, T ukm, T& d1, T& d2, T& d3,
-                                     double eps = 1.0e-8) {
+__device__ inline void rof_flux_ref(T uc, T uip, T uim, T ujp, T ujm, T ukp, T ukm, T& d1, T& d2, T& d3,
+                                    double eps) {
     const T fi = uip - uc, bi = uc - uim, fj = ujp - uc, bj = uc - ujm;
     if (DIM == 3) {
         const T fk = ukp - uc, bk = uc - ukm;
@@ -62,6 +63,68 @@ __device__ inline void rof_flux_math(T uc, T uip, T uim, T ujp, T ujm, T ukp, T 
         d2 = rof_d2<DIM, T>(fi, m[1], T(0), eps);
         d3 = 0;
     }
+}
+
+// The same values.  In-range points take sqrt_in and div_in; one test sends a
+// wave with any other point to rof_flux_ref: a difference that is NaN or
+// overflows (the products and squares are summed: any of them makes the sum NaN
+// or infinite), or a numerator in (0, 2^-100).  Each quotient issues in 26
+// cycles instead of 49, and the minmods need no test of their own (ROF 256^3
+// 84 -> 80 us per iteration, 128^3 13.8 -> 12.7).
+template <int DIM, typename T>
+__device__ inline void rof_flux_math(T uc, T uip, T uim, T ujp, T ujm, T ukp, T ukm, T& d1, T& d2, T& d3,
+                                     double eps = 1.0e-8) {
+    if constexpr (std::is_same<T, float>::value) {
+        const float fi = uip - uc, bi = uc - uim, fj = ujp - uc, bj = uc - ujm;
+        const float ai = __builtin_amdgcn_fmed3f(fi, bi, 0.f), aj = __builtin_amdgcn_fmed3f(fj, bj, 0.f);
+        const float mi = ai * ai, mj = aj * aj;
+        float s1 = fj * fj + mi, s2 = fi * fi + mj, s3 = 0.f, fk = 0.f, sum = __builtin_fmaf(fi, bi, fj * bj);
+        uint32_t key = min_key(tiny_key(fi), tiny_key(fj));
+        if (DIM == 3) {
+            fk = ukp - uc;
+            const float bk = uc - ukm, ak = __builtin_amdgcn_fmed3f(fk, bk, 0.f), mk = ak * ak;
+            s1 = s1 + mk;
+            s2 = s2 + mk;
+            s3 = fk * fk + mj + mi;
+            sum = __builtin_fmaf(fk, bk, sum) + s3;
+            key = min_key(key, tiny_key(fk));
+        }
+        sum = sum + (s1 + s2);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(sum) <= 0x1p+126f) || key < kTinyKey) == 0, 1)) {
+            const double x1 = (double)s1 + eps;
+            const float b1 = DIM == 3 ? (float)sqrt_dn(x1) : sqrt_in((float)x1);
+            const float b2 = sqrt_in((float)((double)s2 + eps));
+            d1 = div_in(fj, b1, rcp_in(b1));
+            d2 = div_in(fi, b2, rcp_in(b2));
+            d3 = 0;
+            if (DIM == 3) {
+                const float b3 = sqrt_in((float)((double)s3 + eps));
+                d3 = div_in(fk, b3, rcp_in(b3));
+            }
+            return;
+        }
+    }
+    rof_flux_ref<DIM, T>(uc, uip, uim, ujp, ujm, ukp, ukm, d1, d2, d3, eps);
+}
+
+// A ring lane's D2 (side) or D1, from the forward difference f along its axis,
+// those across it (fo, bo) and along z: in range as in rof_flux_math.
+template <int DIM>
+__device__ inline float rof_ring_flux(bool side, float f, float fo, float bo, float fk, float bk, double eps) {
+    const float ao = __builtin_amdgcn_fmed3f(fo, bo, 0.f), ak = __builtin_amdgcn_fmed3f(fk, bk, 0.f);
+    const float mo = ao * ao, mk = ak * ak, s = DIM == 3 ? f * f + mo + mk : f * f + mo;
+    const float sum = __builtin_fmaf(fo, bo, __builtin_fmaf(fk, bk, s));
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(sum) <= 0x1p+126f) || tiny_key(f) < kTinyKey) == 0, 1)) {
+        const double x = (double)s + eps;
+        float w = sqrt_in((float)x);
+        if (DIM == 3) {
+            const float w1 = (float)sqrt_dn(x);   // D1's root is rounded from double
+            w = side ? w : w1;
+        }
+        return div_in(f, w, rcp_in(w));
+    }
+    const float no = Mixed<float>::minmod_sq(fo, bo), nk = DIM == 3 ? Mixed<float>::minmod_sq(fk, bk) : 0.f;
+    return side ? rof_d2<DIM, float>(f, no, nk, eps) : rof_d1<DIM, float>(f, no, nk, eps);
 }
 
 // The fluxes D1 (along y), D2 (along x) and, in 3D, D3 (along z) at
@@ -170,15 +233,11 @@ __device__ inline void rof_body(const RofArgs<T>& a, const TileCoord& tc) {
             // only the flux the lane stores: D2 on the column, D1 on the row
             // (the across-difference pair: y for D2, x for D1)
             const T fa = d2lane ? uyp - hc : uxp - hc, ba = d2lane ? hc - uym : hc - uxm;
-            T m[2];
-            Mixed<T>::minmod_sq_n({fa, DIM == 3 ? hp - hc : T(0)}, {ba, DIM == 3 ? hc - hm : T(0)}, m);
-            const T mk = DIM == 3 ? m[1] : T(0);
-            if (d2lane) {
-                const T h2 = rof_d2<DIM, T>(uxp - hc, m[0], mk, 1.0e-8);
-                if (rin) D2l[sy - 1][0] = h2;
-            } else {
-                const T h1 = rof_d1<DIM, T>(uyp - hc, m[0], mk, 1.0e-8);
-                if (rin) D1l[0][sx - 1] = h1;
+            const T q = rof_ring_flux<DIM>(d2lane, (d2lane ? uxp : uyp) - hc, fa, ba, DIM == 3 ? hp - hc : T(0),
+                                           DIM == 3 ? hc - hm : T(0), 1.0e-8);
+            if (rin) {
+                if (d2lane) D2l[sy - 1][0] = q;
+                else D1l[0][sx - 1] = q;
             }
         }
         __syncthreads();
