@@ -297,8 +297,9 @@ __device__ inline float sqrt_rn(float x) {
 // For y in [2^-125, 2^125], v_rcp_f32 followed by one Newton step (two fused
 // multiply-adds) is the correctly rounded reciprocal r (checked for every
 // such float by cilreg_check_rcp_in), and for a = 0 or 2^-100 <= |a| with
-// 2^-60 <= |y| <= 2^64, |a| <= 2^64 the quotient a / y is a r corrected once
-// by its residual (checked by cilreg_check_div_in; all 2^46 pairs of
+// 2^-60 <= |y| <= 2^64, |a| <= 2^64 a quotient a / y that is 0 or a normal number
+// is a r corrected once by its residual (a tie between denormals could round the
+// wrong way: callers bound |y| so that |a| >= 2^-100 gives none; checked by cilreg_check_div_in; all 2^46 pairs of
 // significands give the IEEE quotient, and in that range every step scales
 // with the exponents exactly).  The residual is negated so that a = -0 keeps
 // its sign.  The compiler's IEEE expansion of a / y (two scalings, v_rcp,

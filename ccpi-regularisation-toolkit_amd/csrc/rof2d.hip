@@ -14,31 +14,29 @@ using RofDeepArgs = DeepArgs<float, 1, RofPar>;   // state: u
 
 // The fluxes D1 (along y) and D2 (along x) of N points from u there (uc) and
 // its mirrored neighbours: the values of rof_flux_math<2>.  In-range points
-// take sqrt_in and div_in; one test sends a wave with any other point --
-// a difference that is NaN or overflows (the products and squares are summed:
-// any of them makes the sum NaN or infinite), or a numerator below 2^-100 --
-// to rof_flux_ref.
+// take sqrt_in and div_in; one test sends a wave with any other point (as in
+// rof_flux_math) to rof_flux_ref.
 template <int N>
 __device__ inline void rof2d_fluxes(const float (&uc)[N], const float (&ul)[N], const float (&ur)[N],
                                     const float (&uu)[N], const float (&ud)[N], float (&d1)[N], float (&d2)[N]) {
-    float x1[N], x2[N], sum = 0.0f;
+    float x1[N], x2[N], prod = 0.0f, sq = 0.0f;
     uint32_t key = ~0u;
     #pragma unroll
     for (int r = 0; r < N; ++r) {
         const float fi = ur[r] - uc[r], bi = uc[r] - ul[r], fj = ud[r] - uc[r], bj = uc[r] - uu[r];
         const float mi = __builtin_amdgcn_fmed3f(fi, bi, 0.f), mj = __builtin_amdgcn_fmed3f(fj, bj, 0.f);
         const float s1 = fj * fj + mi * mi, s2 = fi * fi + mj * mj;
-        sum = __builtin_fmaf(fi, bi, sum);
-        sum = __builtin_fmaf(fj, bj, sum);
-        sum = sum + s1;
-        sum = sum + s2;
+        prod = __builtin_fmaf(fi, bi, prod);
+        prod = __builtin_fmaf(fj, bj, prod);
+        sq = sq + s1;
+        sq = sq + s2;
         key = min_key(key, min_key(tiny_key(fi), tiny_key(fj)));
         x1[r] = (float)((double)s1 + 1.0e-8);
         x2[r] = (float)((double)s2 + 1.0e-8);
         d1[r] = fj;
         d2[r] = fi;
     }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(sum) <= 0x1p+126f) || key < kTinyKey) != 0, 0)) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(rof_odd(prod, sq) || key < kTinyKey) != 0, 0)) {
         #pragma unroll
         for (int r = 0; r < N; ++r) {
             float d3;

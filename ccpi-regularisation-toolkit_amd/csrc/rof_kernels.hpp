@@ -65,12 +65,19 @@ __device__ inline void rof_flux_ref(T uc, T uip, T uim, T ujp, T ujm, T ukp, T u
     }
 }
 
+// sq: a sum of squares; prod: a sum of products.  True when sq is not below 2^52
+// or either is NaN or infinite (|prod| adds at most 2^48 otherwise).
+__device__ inline bool rof_odd(float prod, float sq) {
+    return !(__builtin_fmaf(fabsf(prod), 0x1p-80f, sq) < 0x1p+52f);
+}
+
 // The same values.  In-range points take sqrt_in and div_in; one test sends a
-// wave with any other point to rof_flux_ref: a difference that is NaN or
-// overflows (the products and squares are summed: any of them makes the sum NaN
-// or infinite), or a numerator in (0, 2^-100).  Each quotient issues in 26
-// cycles instead of 49, and the minmods need no test of their own (ROF 256^3
-// 84 -> 80 us per iteration, 128^3 13.8 -> 12.7).
+// wave with any other point to rof_flux_ref: sums of squares not below 2^52
+// (with numerators from 2^-100 up every quotient is then a normal number), a
+// product of a minmod's operands that is NaN or infinite, or a numerator in
+// (0, 2^-100).  Each quotient issues in 26 cycles instead of 49, and the minmods
+// need no test of their own (ROF 256^3 84 -> 80 us per iteration, 128^3 13.8 ->
+// 12.7).
 template <int DIM, typename T>
 __device__ inline void rof_flux_math(T uc, T uip, T uim, T ujp, T ujm, T ukp, T ukm, T& d1, T& d2, T& d3,
                                      double eps = 1.0e-8) {
@@ -78,7 +85,7 @@ __device__ inline void rof_flux_math(T uc, T uip, T uim, T ujp, T ujm, T ukp, T 
         const float fi = uip - uc, bi = uc - uim, fj = ujp - uc, bj = uc - ujm;
         const float ai = __builtin_amdgcn_fmed3f(fi, bi, 0.f), aj = __builtin_amdgcn_fmed3f(fj, bj, 0.f);
         const float mi = ai * ai, mj = aj * aj;
-        float s1 = fj * fj + mi, s2 = fi * fi + mj, s3 = 0.f, fk = 0.f, sum = __builtin_fmaf(fi, bi, fj * bj);
+        float s1 = fj * fj + mi, s2 = fi * fi + mj, s3 = 0.f, fk = 0.f, prod = __builtin_fmaf(fi, bi, fj * bj);
         uint32_t key = min_key(tiny_key(fi), tiny_key(fj));
         if (DIM == 3) {
             fk = ukp - uc;
@@ -86,11 +93,11 @@ __device__ inline void rof_flux_math(T uc, T uip, T uim, T ujp, T ujm, T ukp, T 
             s1 = s1 + mk;
             s2 = s2 + mk;
             s3 = fk * fk + mj + mi;
-            sum = __builtin_fmaf(fk, bk, sum) + s3;
+            prod = __builtin_fmaf(fk, bk, prod);
             key = min_key(key, tiny_key(fk));
         }
-        sum = sum + (s1 + s2);
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(sum) <= 0x1p+126f) || key < kTinyKey) == 0, 1)) {
+        const bool odd = rof_odd(prod, s1 + s2 + s3) || key < kTinyKey;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) == 0, 1)) {
             const double x1 = (double)s1 + eps;
             const float b1 = DIM == 3 ? (float)sqrt_dn(x1) : sqrt_in((float)x1);
             const float b2 = sqrt_in((float)((double)s2 + eps));
@@ -113,8 +120,8 @@ template <int DIM>
 __device__ inline float rof_ring_flux(bool side, float f, float fo, float bo, float fk, float bk, double eps) {
     const float ao = __builtin_amdgcn_fmed3f(fo, bo, 0.f), ak = __builtin_amdgcn_fmed3f(fk, bk, 0.f);
     const float mo = ao * ao, mk = ak * ak, s = DIM == 3 ? f * f + mo + mk : f * f + mo;
-    const float sum = __builtin_fmaf(fo, bo, __builtin_fmaf(fk, bk, s));
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(sum) <= 0x1p+126f) || tiny_key(f) < kTinyKey) == 0, 1)) {
+    const bool odd = rof_odd(__builtin_fmaf(fo, bo, fk * bk), s) || tiny_key(f) < kTinyKey;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) == 0, 1)) {
         const double x = (double)s + eps;
         float w = sqrt_in((float)x);
         if (DIM == 3) {

@@ -267,7 +267,7 @@ int tgv_solve_2d(const float* d_f, float* d_out, float lambda, float alpha1, flo
     k.alpha0 = alpha0;
     k.lt = lambda + k.tau;
     auto in = [](float v) { return v >= 0x1p-30f && v <= 0x1p+30f; };
-    k.fast = in(alpha1) && in(alpha0) && in(k.lt);
+    k.fast = in(alpha1) && in(alpha0) && in(k.lt) && k.lt <= 0x1p+26f;   // quotients by lt stay normal
     k.ra1 = 1.0f / alpha1;
     k.ra0 = 1.0f / alpha0;
     k.rlt = 1.0f / k.lt;
