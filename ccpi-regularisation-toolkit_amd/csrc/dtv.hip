@@ -608,8 +608,8 @@ static void launch_dtv(const DtvArgs<T>& a, bool iso, bool small, hipStream_t s)
     }
 }
 
-// Device-resident FGP-dTV solve; volumes that deep3_fits accepts run on
-// dtv_solve_3d unless opts.depth == 1.  d_out receives D of the final iteration
+// Device-resident FGP-dTV solve; unless opts.depth == 1, images run on
+// dtv_solve_2d and volumes that deep3_fits accepts on dtv_solve_3d.  d_out receives D of the final iteration
 // (left untouched when iter == 0); with epsil != 0 its prior contents seed the
 // first residual (FGP_dTV_core.c:78,131).
 template <typename T>
@@ -645,6 +645,15 @@ int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsi
                                B[2], eta, nx, ny, nz);
     };
     if constexpr (std::is_same<T, float>::value) {
+        if (dim == 2 && opts.depth != 1) {
+            Arena ar;
+            const size_t o0 = ar.reserve(n * sizeof(float)), o1 = ar.reserve(n * sizeof(float));
+            if (ar.allocate() != 0) return -1;
+            float* const B[3] = {(float*)ar.at(o0), (float*)ar.at(o1), (float*)ar.at(o1)};
+            refgrad(B);
+            return dtv_solve_2d(d_f, {B[0], B[1]}, d_out, lambda, iter, epsil, method, nonneg, nx, ny, mult, opts, s,
+                                iters_done, re);
+        }
         // Checked passes have two levels (three spill), which pay unless the
         // fields stream from HBM in rows of whole 128-byte lines, the tiled
         // pass's best case: 256^3 checked every fifth iteration 157 us tiled and

@@ -66,6 +66,14 @@ int fgp_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float e
 template <typename S>
 int fgp_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float epsil, int method, int nonneg, int nx,
                  int ny, int nz, const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws);
+int sb_solve_2d(const float* d_f, float* d_out, float lam, float mu, float nc, float thr, int iter, float epsil,
+                int method, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re,
+                const WarmState* ws);
+int ndf_solve_2d(const float* d_f, float* d_out, float lambda, float sigma, int iter, float tau, int penalty,
+                 float epsil, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re);
+int dtv_solve_2d(const float* d_f, const float* const (&B)[2], float* d_out, float lambda, int iter, float epsil,
+                 int method, int nonneg, int nx, int ny, const std::vector<float>& mult, const Opts& opts,
+                 hipStream_t s, int* iters_done, float* re);
 int dtv_solve_3d(const float* d_f, const float* const (&B)[3], float* d_out, float lambda, int iter, float epsil,
                  int method, int nonneg, int nx, int ny, int nz, const std::vector<float>& mult, const Opts& opts,
                  hipStream_t s, int* iters_done, float* re);
