@@ -520,6 +520,13 @@ int sb_solve(const T* d_f, T* d_out, T mu_in, int iter, T epsil, int method, int
         CILREG_CK(hipStreamSynchronize(s));
         return 0;
     }
+    // constants in the working precision (SB_TV_core.c:45-46, :153, :179, :258)
+    const T mu = (T)1 / mu_in;
+    const T lam = (T)2 * mu;
+    const T nc = (T)1 / (mu + (dim == 3 ? (T)6 : (T)4) * lam);
+    const T thr = (T)1 / lam;
+    if (dim == 2 && opts.depth != 1 && nx > 1 && ny > 1)
+        return sb_solve_2d(d_f, d_out, lam, mu, nc, thr, iter, epsil, method, nx, ny, opts, s, iters_done, re, ws);
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T));
     const bool aniso = method == 1;
     // one fused pass per iteration, unless the last tile is one column / row
@@ -569,11 +576,6 @@ int sb_solve(const T* d_f, T* d_out, T mu_in, int iter, T epsil, int method, int
     }
     Ctrl* ctrl = (Ctrl*)ar.at(oCtrl);
     double* partials = (double*)ar.at(oPart);
-    // constants in the working precision (SB_TV_core.c:45-46, :153, :179, :258)
-    const T mu = (T)1 / mu_in;
-    const T lam = (T)2 * mu;
-    const T nc = (T)1 / (mu + (dim == 3 ? (T)6 : (T)4) * lam);
-    const T thr = (T)1 / lam;
     auto step = [&](int k, bool check) {
         SbArgs<T> a;
         const int cur = k & 1, nxt = cur ^ 1;

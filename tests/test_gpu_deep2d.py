@@ -16,7 +16,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-METHODS = ["rof", "fgp", "pd", "tgv", "dtv"]
+METHODS = ["rof", "fgp", "pd", "tgv", "dtv", "sb"]
 PRECISION = {"fgp": ["fp32", "bf16", "fp16"], "pd": ["fp32", "bf16", "fp16"], "tgv": ["fp32", "bf16", "fp16"],
              "rof": ["fp32"]}
 SHAPES = [(2, 2), (1, 65), (33, 1), (2, 300), (31, 33), (32, 32), (33, 64), (64, 65), (129, 63), (65, 200),
@@ -119,7 +119,7 @@ def test_values_outside_the_fast_ranges(method):
         _same(_run(method, y, 11, nonneg=0, depth=1), _run(method, y, 11, nonneg=0), f"{method} {bad}")
 
 
-@pytest.mark.parametrize("method", ["fgp", "pd", "tgv"])
+@pytest.mark.parametrize("method", ["fgp", "pd", "tgv", "sb"])
 def test_warm_start_across_passes(method):
     from ccpi.filters import device as D
     x = _vol((100, 131), 8)
