@@ -16,7 +16,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-METHODS = ["rof", "fgp", "pd", "tgv", "dtv", "sb"]
+METHODS = ["rof", "fgp", "pd", "tgv", "dtv", "sb"] + [f"ndf{p}" for p in range(6)]
 PRECISION = {"fgp": ["fp32", "bf16", "fp16"], "pd": ["fp32", "bf16", "fp16"], "tgv": ["fp32", "bf16", "fp16"],
              "rof": ["fp32"]}
 SHAPES = [(2, 2), (1, 65), (33, 1), (2, 300), (31, 33), (32, 32), (33, 64), (64, 65), (129, 63), (65, 200),
