@@ -30,11 +30,43 @@ struct TgvArgs {
 // and the +y neighbour (along y).
 enum { L_P1, L_P2, L_Q11, L_Q22, L_Q12, L_Q13, L_Q23, L_N };
 
+// sqrt(ss) / alpha, the norm a projection compares with 1.
+//
+// 3D with 16-bit storage (which HBM does not bound): a wave whose points all lie
+// inside the ball -- ss below 0.999 alpha^2, for an alpha whose square is a
+// normal number; NaN and infinity fail it -- returns 0 without the root and the
+// division.  Few points leave their balls: 256^3 bf16 212 -> 198 us per iteration,
+// 190 x 257 x 231 195 -> 183.
+//
+// 3D FP32: that branch gains nothing (256^3 258 against 257-266), and the
+// 80-VGPR pass answers to the order of its instructions: the root by v_sqrt_f32
+// and its two neighbours' residuals (sqrtf's bits on [2^-96, FLT_MAX]) is 1-2%
+// faster there than sqrt_rn's form (192 x 512 x 512 761 against 777 us).
+template <int DIM, typename T, typename S>
+__device__ inline T tgv_norm(T ss, T alpha) {
+    if constexpr (DIM == 3 && sizeof(S) == 2) {
+        const T lim = alpha >= (T)0x1p-60f ? (T)0.999f * (alpha * alpha) : (T)0;
+        if (!__builtin_amdgcn_ballot_w64(!(ss < lim))) return (T)0;
+        return dsqrt(ss) / alpha;
+    } else if constexpr (DIM == 3 && std::is_same<S, float>::value) {
+        const bool fast = ss >= 0x1p-96f && ss <= 0x1.fffffep127f;   // false for NaN
+        if (__builtin_amdgcn_ballot_w64(!fast)) return sqrtf(ss) / alpha;
+        const float r = __builtin_amdgcn_sqrtf(ss);
+        const uint32_t ri = __float_as_uint(r);
+        const float rm = __uint_as_float(ri - 1u), rp = __uint_as_float(ri + 1u);
+        const uint32_t above_m = __float_as_uint(__builtin_fmaf(rm, r, -ss)) >> 31;   // 1: ss - (r - 1 ulp) r > 0
+        const uint32_t above_p = __float_as_uint(__builtin_fmaf(rp, r, -ss)) >> 31;
+        return __uint_as_float(ri - 1u + above_m + above_p) / alpha;
+    } else {
+        return dsqrt(ss) / alpha;
+    }
+}
+
 // The dual step at one point (TGV_core.c:351-446): P and Q of the next
 // iterate from the old P, Q there, u_bar and v_bar there (u, v) and at the
 // +x / +y / +z neighbours, and whether the point is the last along each axis
 // (the forward difference is zero there).  Shared by every TGV kernel.
-template <int DIM, typename T>
+template <int DIM, typename T, typename S>
 __device__ inline void tgv_dual_math(T sigma, T alpha1, T alpha0, bool lx, bool ly, bool lz, T u, const T v[3], T ux,
                                      T uy, T uz, const T vx[3], const T vy[3], const T vz[3], const T po[3],
                                      const T qo[6], T p[3], T q[6]) {
@@ -44,10 +76,10 @@ __device__ inline void tgv_dual_math(T sigma, T alpha1, T alpha0, bool lx, bool 
     T nrm;
     if (DIM == 3) {
         p[2] = po[2] + sigma * (lz ? -v[2] : (uz - u) - v[2]);
-        nrm = dsqrt(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]) / alpha1;
+        nrm = tgv_norm<DIM, T, S>(p[0] * p[0] + p[1] * p[1] + p[2] * p[2], alpha1);
     } else {
         p[2] = 0;
-        nrm = dsqrt(p[0] * p[0] + p[1] * p[1]) / alpha1;
+        nrm = tgv_norm<DIM, T, S>(p[0] * p[0] + p[1] * p[1], alpha1);
     }
     if (nrm > (T)1) {
         p[0] /= nrm;
@@ -71,9 +103,9 @@ __device__ inline void tgv_dual_math(T sigma, T alpha1, T alpha0, bool lx, bool 
         q[3] = qo[3] + sigma * ((T)0.5 * (d[1][0] + d[0][1]));
         q[4] = qo[4] + sigma * ((T)0.5 * (d[2][0] + d[0][2]));
         q[5] = qo[5] + sigma * ((T)0.5 * (d[2][1] + d[1][2]));
-        T m = dsqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + (T)2 * q[3] * q[3] + (T)2 * q[4] * q[4] +
-                    (T)2 * q[5] * q[5]);
-        m = m / alpha0;
+        const T m = tgv_norm<DIM, T, S>(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + (T)2 * q[3] * q[3] +
+                                            (T)2 * q[4] * q[4] + (T)2 * q[5] * q[5],
+                                        alpha0);
         if (m > (T)1) {
             #pragma unroll
             for (int c = 0; c < 6; ++c) q[c] /= m;
@@ -132,7 +164,7 @@ __device__ inline void tgv_dual_at(const TgvArgs<T, S>& a, int px, int py, int z
         ldpair<T>(a.P[0], i, po[0], po[1]);
         ldpair<T>(a.Q[0], i, qo[0], qo[1]);
         qo[2] = ldx<T>(a.Q[2], i);
-        tgv_dual_math<DIM, T>(a.sigma, a.alpha1, a.alpha0, lx, ly, lz, u, v, ux, uy, uz, vx, vy, vz, po, qo, p, q);
+        tgv_dual_math<DIM, T, S>(a.sigma, a.alpha1, a.alpha0, lx, ly, lz, u, v, ux, uy, uz, vx, vy, vz, po, qo, p, q);
         return;
     }
     if constexpr (tgv_pairs<DIM, S>() && DIM == 3) {
@@ -157,7 +189,7 @@ __device__ inline void tgv_dual_at(const TgvArgs<T, S>& a, int px, int py, int z
         ldpair<T>(a.Q[0], i, qo[0], qo[1]);
         ldpair<T>(a.Q[2], i, qo[2], qo[3]);
         ldpair<T>(a.Q[4], i, qo[4], qo[5]);
-        tgv_dual_math<DIM, T>(a.sigma, a.alpha1, a.alpha0, lx, ly, lz, u, v, ux, uy, uz, vx, vy, vz, po, qo, p, q);
+        tgv_dual_math<DIM, T, S>(a.sigma, a.alpha1, a.alpha0, lx, ly, lz, u, v, ux, uy, uz, vx, vy, vz, po, qo, p, q);
         return;
     }
     if (!carried) {
@@ -178,7 +210,7 @@ __device__ inline void tgv_dual_at(const TgvArgs<T, S>& a, int px, int py, int z
     const int nq = DIM == 3 ? 6 : 3;
     #pragma unroll
     for (int c = 0; c < nq; ++c) qo[c] = ldx<T>(a.Q[c], i);
-    tgv_dual_math<DIM, T>(a.sigma, a.alpha1, a.alpha0, lx, ly, lz, u, v, ux, uy, uz, vx, vy, vz, po, qo, p, q);
+    tgv_dual_math<DIM, T, S>(a.sigma, a.alpha1, a.alpha0, lx, ly, lz, u, v, ux, uy, uz, vx, vy, vz, po, qo, p, q);
 }
 
 // Stores the state of one point (u_bar, v_bar, P, Q) at element i.
@@ -626,7 +658,7 @@ __device__ inline void tgv2_body(const Tgv2Args<T, S>& a, const TileCoord& tc) {
                     #pragma unroll
                     for (int c = 0; c < 6; ++c) qo[c] = through_storage<T, S>(q1v[s][c]);
                     const bool bl_x = X[s] == g.nx - 1, bl_y = Y[s] == g.ny - 1, bl_z = zc == nz - 1;
-                    tgv_dual_math<3, T>(sigma, a.alpha1, a.alpha0, bl_x, bl_y, bl_z, u, v, ux, uy, uz, vx, vy, vz,
+                    tgv_dual_math<3, T, S>(sigma, a.alpha1, a.alpha0, bl_x, bl_y, bl_z, u, v, ux, uy, uz, vx, vy, vz,
                                         po, qo, p2[s], q2[s]);
                     PQ[L_P1][by[s]][bx[s]] = p2[s][0];
                     PQ[L_P2][by[s]][bx[s]] = p2[s][1];
