@@ -22,16 +22,19 @@ using TgvDeepArgs = DeepArgs<float, 8, TgvPar>;
 // components, ss their (weighted) sum of squares.  |v| / alpha > 1 decides as
 // in the reference: below 2^-90 the sum is raised to it, where the quotient is
 // far under 1 (fast: alpha >= 2^-30).  A point inside the ball divides by 1,
-// which leaves it as it is.  A wave with a sum above lim, or with a component
-// in (0, 2^-100) that is really divided, takes the reference's expressions.
+// which leaves it as it is.  A wave with a sum above lim or NaN (a point that
+// holds an infinity beside a NaN keeps it: the reference scales nothing there,
+// and div_in would turn it into a NaN), or with a component in (0, 2^-100) that
+// is really divided, takes the reference's expressions.  One test serves the N
+// sums: their total is NaN if one is, and above lim if one is.
 template <int NC, int N>
 __device__ inline bool tgv2d_ball(float (&v)[NC][N], const float (&ss)[N], float alpha, float ra, float lim,
                                   bool fast) {
-    float n[N], top = 0.0f;
+    float n[N], total = 0.0f;
     bool odd = !fast;
     #pragma unroll
     for (int r = 0; r < N; ++r) {
-        top = __builtin_fmaxf(top, ss[r]);
+        total = total + ss[r];
         const float w = sqrt_in(__builtin_fmaxf(ss[r], 0x1p-90f));
         const float m = div_in(w, alpha, ra);
         n[r] = __builtin_fmaxf(m, 1.0f);
@@ -40,7 +43,7 @@ __device__ inline bool tgv2d_ball(float (&v)[NC][N], const float (&ss)[N], float
         for (int c = 1; c < NC; ++c) key = min_key(key, tiny_key(v[c][r]));
         odd = odd || (key < kTinyKey && m > 1.0f);
     }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd || top > lim) != 0, 0)) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd || !(total <= lim)) != 0, 0)) {
         #pragma unroll
         for (int r = 0; r < N; ++r) {
             const float m = sqrtf(ss[r]) / alpha;
