@@ -22,6 +22,7 @@
 #pragma once
 #include "runtime.hpp"
 #include "state.hpp"
+#include <functional>
 
 namespace cilreg {
 
@@ -218,6 +219,15 @@ void deep_dispatch(int s, Fn&& fn) {
     }
 }
 
+// Fields of a solve's own beside its state (FGP-dTV's B): they lie in the
+// solve's allocation, so that no kernel is queued before the last allocation
+// that can fail (a block given back while a kernel still writes it could reach
+// another thread's solve).  fill queues the kernels that compute them.
+struct DeepExtra {
+    int fields;   // at most 3, float
+    std::function<void(float* const (&)[3])> fill;
+};
+
 // ---------------------------------------------------------------------------
 // the solve loop
 // ---------------------------------------------------------------------------
@@ -241,7 +251,8 @@ void deep_dispatch(int s, Fn&& fn) {
 // that overlaps the input, which later regions of the same pass still read.
 template <class M, typename T>
 int deep_solve(M& m, const T* d_f, T* d_out, int nx, int ny, int iter, T epsil, const Opts& opts, hipStream_t s,
-               int* iters_done, float* re, const WarmState* ws, int* last_iter = nullptr) {
+               int* iters_done, float* re, const WarmState* ws, int* last_iter = nullptr,
+               const DeepExtra* extra = nullptr) {
     const size_t n = (size_t)nx * ny;
     const bool use_tol = epsil != (T)0;
     int most = opts.depth >= 2 ? 2 : kDeepMax;
@@ -251,14 +262,16 @@ int deep_solve(M& m, const T* d_f, T* d_out, int nx, int ny, int iter, T epsil, 
 
     Arena ar;
     if (opts.scratch) ar.use_external(opts.scratch, opts.scratch_bytes);
-    size_t of[2][M::NF], oR = 0;
+    size_t of[2][M::NF], oX[3] = {0, 0, 0}, oR = 0;
     for (int b = 0; b < 2; ++b)
         for (int i = 0; i < M::NF; ++i) of[b][i] = ar.reserve(n * m.field_size(i));
+    for (int i = 0; extra && i < extra->fields; ++i) oX[i] = ar.reserve(n * sizeof(float));
     const bool apart = d_out + n <= d_f || d_f + n <= d_out;
     if (!apart) oR = ar.reserve(n * sizeof(T));
     const size_t oCtrl = ar.reserve(sizeof(Ctrl));
     const size_t oPart = ar.reserve((size_t)plan.g.nblocks * 2 * width * sizeof(double));
     if (ar.allocate() != 0) return -1;
+    if (extra) extra->fill({(float*)ar.at(oX[0]), (float*)ar.at(oX[1]), (float*)ar.at(oX[2])});
     T* res = apart ? d_out : (T*)ar.at(oR);
     Ctrl* ctrl = (Ctrl*)ar.at(oCtrl);
     const bool warm = ws && ws->warm;

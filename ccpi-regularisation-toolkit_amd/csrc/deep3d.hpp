@@ -165,7 +165,8 @@ struct Deep3Args {
 // and launch(T, shape, args, stream).
 template <class M>
 int deep3_solve(M& m, const float* d_f, float* d_out, int nx, int ny, int nz, int iter, float epsil, const Opts& opts,
-                hipStream_t s, int* iters_done, float* re, const WarmState* ws, int* last_iter = nullptr) {
+                hipStream_t s, int* iters_done, float* re, const WarmState* ws, int* last_iter = nullptr,
+                const DeepExtra* extra = nullptr) {
     const size_t n = (size_t)nx * ny * nz;
     const bool use_tol = epsil != 0.0f;
     const int most = std::min(iter, m.most(use_tol));
@@ -173,7 +174,8 @@ int deep3_solve(M& m, const float* d_f, float* d_out, int nx, int ny, int nz, in
     const Deep3Plan plan = plan_deep3(nx, ny, nz, M::rlo, M::rhi, m.cost(), m.bytes(), most, opts.zchunk);
     const int width = plan.T;
     Arena ar;
-    size_t of[2][M::NF], oR = 0;
+    size_t of[2][M::NF], oX[3] = {0, 0, 0}, oR = 0;
+    for (int i = 0; extra && i < extra->fields; ++i) oX[i] = ar.reserve(n * sizeof(float) + kFieldSkew);
     for (int b = 0; b < 2; ++b)
         for (int i = 0; i < M::NF; ++i) of[b][i] = ar.reserve(n * m.field_size(i) + kFieldSkew);
     const bool apart = d_out + n <= d_f || d_f + n <= d_out;
@@ -181,6 +183,7 @@ int deep3_solve(M& m, const float* d_f, float* d_out, int nx, int ny, int nz, in
     const size_t oCtrl = ar.reserve(sizeof(Ctrl));
     const size_t oPart = ar.reserve((size_t)plan.g.nblocks * 2 * width * sizeof(double));
     if (ar.allocate() != 0) return -1;
+    if (extra) extra->fill({(float*)ar.at(oX[0]), (float*)ar.at(oX[1]), (float*)ar.at(oX[2])});
     float* res = apart ? d_out : (float*)ar.at(oR);
     Ctrl* ctrl = (Ctrl*)ar.at(oCtrl);
     const bool warm = ws && ws->warm;

@@ -645,30 +645,17 @@ int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsi
                                B[2], eta, nx, ny, nz);
     };
     if constexpr (std::is_same<T, float>::value) {
-        if (dim == 2 && opts.depth != 1) {
-            Arena ar;
-            const size_t o0 = ar.reserve(n * sizeof(float)), o1 = ar.reserve(n * sizeof(float));
-            if (ar.allocate() != 0) return -1;
-            float* const B[3] = {(float*)ar.at(o0), (float*)ar.at(o1), (float*)ar.at(o1)};
-            refgrad(B);
-            return dtv_solve_2d(d_f, {B[0], B[1]}, d_out, lambda, iter, epsil, method, nonneg, nx, ny, mult, opts, s,
+        if (dim == 2 && opts.depth != 1)
+            return dtv_solve_2d(d_f, refgrad, d_out, lambda, iter, epsil, method, nonneg, nx, ny, mult, opts, s,
                                 iters_done, re);
-        }
         // Checked passes have two levels (three spill), which pay unless the
         // fields stream from HBM in rows of whole 128-byte lines, the tiled
         // pass's best case: 256^3 checked every fifth iteration 157 us tiled and
         // 176 in registers, 190 x 257 x 231 163 and 105, 128^3 25.6 and 22.2.
         const bool tiled = epsil != (T)0 && nx % 32 == 0 && n * 64 > kDeep3CacheBytes;
-        if (dim == 3 && opts.depth != 1 && deep3_fits(nx, ny, nz) && !tiled) {
-            Arena ar;
-            size_t oB[3];
-            for (size_t& o : oB) o = ar.reserve(n * sizeof(float) + kFieldSkew);
-            if (ar.allocate() != 0) return -1;
-            float* const B[3] = {(float*)ar.at(oB[0]), (float*)ar.at(oB[1]), (float*)ar.at(oB[2])};
-            refgrad(B);
-            return dtv_solve_3d(d_f, {B[0], B[1], B[2]}, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, mult,
-                                opts, s, iters_done, re);
-        }
+        if (dim == 3 && opts.depth != 1 && deep3_fits(nx, ny, nz) && !tiled)
+            return dtv_solve_3d(d_f, refgrad, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, mult, opts, s,
+                                iters_done, re);
     }
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;

@@ -215,8 +215,8 @@ int fgp_solve_2d(const float* d_f, float* d_out, float lambda, int iter, float e
     return 0;
 }
 
-// FGP-dTV; B is dtv_solve's, mult the t_k sequence's factors.
-int dtv_solve_2d(const float* d_f, const float* const (&B)[2], float* d_out, float lambda, int iter, float epsil,
+// FGP-dTV; refgrad queues the kernel that computes B, mult holds the t_k sequence's factors.
+int dtv_solve_2d(const float* d_f, const RefGrad& refgrad, float* d_out, float lambda, int iter, float epsil,
                  int method, int nonneg, int nx, int ny, const std::vector<float>& mult, const Opts& opts,
                  hipStream_t s, int* iters_done, float* re) {
     FgpDeep<float, true> m;
@@ -225,9 +225,12 @@ int dtv_solve_2d(const float* d_f, const float* const (&B)[2], float* d_out, flo
     m.nonneg = nonneg != 0;
     m.iso = method == 0;
     m.mult = mult;
-    m.B[0] = B[0];
-    m.B[1] = B[1];
-    return deep_solve(m, d_f, d_out, nx, ny, iter, epsil, opts, s, iters_done, re, nullptr);
+    const DeepExtra b{2, [&](float* const (&B)[3]) {
+        m.B[0] = B[0];
+        m.B[1] = B[1];
+        refgrad({B[0], B[1], B[1]});   // two components
+    }};
+    return deep_solve(m, d_f, d_out, nx, ny, iter, epsil, opts, s, iters_done, re, nullptr, nullptr, &b);
 }
 
 template int fgp_solve_2d<float>(const float*, float*, float, int, float, int, int, int, int, const Opts&, hipStream_t,

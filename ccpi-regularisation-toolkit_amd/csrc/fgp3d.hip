@@ -378,18 +378,21 @@ int fgp_solve_3d(const float* d_f, float* d_out, float lambda, int iter, float e
     return 0;
 }
 
-// FGP-dTV; B is dtv_solve's, mult the t_k sequence's factors.
-int dtv_solve_3d(const float* d_f, const float* const (&B)[3], float* d_out, float lambda, int iter, float epsil,
+// FGP-dTV (arguments as dtv_solve_2d's).
+int dtv_solve_3d(const float* d_f, const RefGrad& refgrad, float* d_out, float lambda, int iter, float epsil,
                  int method, int nonneg, int nx, int ny, int nz, const std::vector<float>& mult, const Opts& opts,
                  hipStream_t s, int* iters_done, float* re) {
     Fgp3<float, true> m;
     m.par.lambda = lambda;
     m.par.step = 1.0f / (26.0f * lambda);
     m.par.nonneg = nonneg != 0;
-    for (int c = 0; c < 3; ++c) m.par.B[c] = B[c];
     m.iso = method == 0;
     m.mult = mult;
-    return deep3_solve(m, d_f, d_out, nx, ny, nz, iter, epsil, opts, s, iters_done, re, nullptr);
+    const DeepExtra b{3, [&](float* const (&B)[3]) {
+        for (int c = 0; c < 3; ++c) m.par.B[c] = B[c];
+        refgrad(B);
+    }};
+    return deep3_solve(m, d_f, d_out, nx, ny, nz, iter, epsil, opts, s, iters_done, re, nullptr, nullptr, &b);
 }
 
 template int fgp_solve_3d<float>(const float*, float*, float, int, float, int, int, int, int, int, const Opts&,

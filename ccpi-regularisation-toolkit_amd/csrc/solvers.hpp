@@ -11,6 +11,7 @@
 #pragma once
 #include "runtime.hpp"
 #include "state.hpp"
+#include <functional>
 
 namespace cilreg {
 
@@ -71,10 +72,12 @@ int sb_solve_2d(const float* d_f, float* d_out, float lam, float mu, float nc, f
                 const WarmState* ws);
 int ndf_solve_2d(const float* d_f, float* d_out, float lambda, float sigma, int iter, float tau, int penalty,
                  float epsil, int nx, int ny, const Opts& opts, hipStream_t s, int* iters_done, float* re);
-int dtv_solve_2d(const float* d_f, const float* const (&B)[2], float* d_out, float lambda, int iter, float epsil,
+// Queues the kernel that fills the components of FGP-dTV's B.
+using RefGrad = std::function<void(float* const (&)[3])>;
+int dtv_solve_2d(const float* d_f, const RefGrad& refgrad, float* d_out, float lambda, int iter, float epsil,
                  int method, int nonneg, int nx, int ny, const std::vector<float>& mult, const Opts& opts,
                  hipStream_t s, int* iters_done, float* re);
-int dtv_solve_3d(const float* d_f, const float* const (&B)[3], float* d_out, float lambda, int iter, float epsil,
+int dtv_solve_3d(const float* d_f, const RefGrad& refgrad, float* d_out, float lambda, int iter, float epsil,
                  int method, int nonneg, int nx, int ny, int nz, const std::vector<float>& mult, const Opts& opts,
                  hipStream_t s, int* iters_done, float* re);
 template <typename S>

@@ -35,3 +35,27 @@ def test_tgv_image_with_adjacent_infinities(pair, precision):
     for iters in (1, 2, 7, 9):
         _same(D.tgv(x, 0.05, 1.3, 1.7, iters, 12.0, precision=precision, depth=1),
               D.tgv(x, 0.05, 1.3, 1.7, iters, 12.0, precision=precision), f"{pair} iters={iters}")
+
+
+@pytest.mark.parametrize("shape", [(70, 90), (60, 95, 100)], ids=str)
+def test_dtv_allocates_once(shape):
+    """All of an FGP-dTV solve's memory is one allocation ahead of its first
+    kernel: a second one that failed would hand the first back to the pool with
+    the reference gradient's kernel still writing it."""
+    import ctypes
+    from ccpi.filters import device as D
+    from ccpi.filters.utils import require_gpu_lib
+    lib = require_gpu_lib()
+    lib.cilreg_inject_alloc_failure.argtypes = [ctypes.c_int]
+    lib.cilreg_inject_alloc_failure.restype = None
+    x, ref = _vol(shape, 4), _vol(shape, 5)
+    want = D.dtv(x, ref, 0.03, 9, depth=1)
+    try:
+        lib.cilreg_inject_alloc_failure(1)
+        with pytest.raises(RuntimeError, match="alloc"):
+            D.dtv(x, ref, 0.03, 9)
+        lib.cilreg_inject_alloc_failure(2)   # there is no second allocation to fail
+        got = D.dtv(x, ref, 0.03, 9)
+    finally:
+        lib.cilreg_inject_alloc_failure(0)
+    _same(got, want, f"{shape}")
