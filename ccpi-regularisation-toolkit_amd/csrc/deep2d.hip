@@ -13,7 +13,9 @@ DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[
         const int h = 64 * c.nw / c.lx * c.r;
         for (int w = 1; w <= most; ++w) {
             const int lo = rlo * w, hi = rhi * w;
-            if (w > 1 && (c.lx - lo - hi < 8 || h - lo - hi < 4)) break;
+            // what the inner edges leave of a region (the low ones have none along y)
+            const bool rows = h < 32 ? ny <= h : w == 1 || h - lo - hi >= 4;
+            if (!rows || (w > 1 && c.lx - lo - hi < 8)) break;
             const Deep2D g = make_deep(nx, ny, c.lx, h, lo, hi);
             // workgroups per CU: whole rounds while few, then about the mean
             const double per = g.nblocks / kCus, load = per <= 4 ? ceil(per) : per + 0.5;

@@ -195,6 +195,13 @@ constexpr DeepShapeCost kDeepShapes[] = {
     {64, 16, 2, 3.4},   // 64 x 32
     {64, 16, 4, 4.4},   // 64 x 64: least overlap
     {64, 8, 4, 3.7},    // 64 x 32 on half the waves: several regions per CU
+    // 64 x 4 and 64 x 8: images of so few rows.  Long ones would leave 3/4 and
+    // more of the others empty, which is slower than the one-iteration kernels'
+    // 64 x 4 tiles (10^6 x 4, us per iteration by tiles, in 64 x 32 regions and
+    // here: FGP 26.4, 35.7, 9.0; TGV 58, 109, 18; ROF 28, 56, 12; 10^6 x 8: FGP
+    // 51, 37, 13.5; TGV with BF16 storage 92, 129, 33).
+    {64, 4, 1, 3.1},
+    {64, 4, 2, 3.1},
 };
 constexpr int kDeepShapeCount = (int)(sizeof(kDeepShapes) / sizeof(kDeepShapes[0]));
 
@@ -215,7 +222,9 @@ void deep_dispatch(int s, Fn&& fn) {
         case 0: fn(DeepShape<32, 16, 1>{}); break;
         case 1: fn(DeepShape<64, 16, 2>{}); break;
         case 2: fn(DeepShape<64, 16, 4>{}); break;
-        default: fn(DeepShape<64, 8, 4>{}); break;
+        case 3: fn(DeepShape<64, 8, 4>{}); break;
+        case 4: fn(DeepShape<64, 4, 1>{}); break;
+        default: fn(DeepShape<64, 4, 2>{}); break;
     }
 }
 

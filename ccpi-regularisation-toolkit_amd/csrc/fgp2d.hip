@@ -163,7 +163,8 @@ template <typename S, bool DIR = false>
 struct FgpDeep {
     using Args = FgpDeepArgs;
     static constexpr int NF = 4, rlo = 1, rhi = 1, words = DIR ? 11 : 9;
-    static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.52, 0.42}, {0.70, 0.72}, {1.08, 1.15}, {0.72, 0.50}};
+    static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.52, 0.42}, {0.70, 0.72}, {1.08, 1.15}, {0.72, 0.50}, {0.50, 0.085},
+                                                              {0.55, 0.12}};
     static constexpr bool seeded = true;
     float lambda, step;
     int nonneg;

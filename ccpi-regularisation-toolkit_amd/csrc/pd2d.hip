@@ -118,7 +118,8 @@ template <typename S>
 struct PdDeep {
     using Args = PdDeepArgs;
     static constexpr int NF = 3, rlo = 1, rhi = 1, words = 7;
-    static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.53, 0.48}, {0.85, 0.82}, {1.40, 1.70}, {0.85, 0.70}};
+    static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.53, 0.48}, {0.85, 0.82}, {1.40, 1.70}, {0.85, 0.70}, {0.50, 0.09},
+                                                              {0.55, 0.12}};
     static constexpr bool seeded = false;
     PdPar par;
     bool iso;

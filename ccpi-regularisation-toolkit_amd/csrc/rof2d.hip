@@ -159,7 +159,8 @@ struct RofDeep {
     using Args = RofDeepArgs;
     // D1, D2 at the low neighbours read u two columns / rows away
     static constexpr int NF = 1, rlo = 2, rhi = 1, words = 3;
-    static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.75, 0.61}, {1.12, 1.00}, {1.95, 1.70}, {1.30, 0.86}};
+    static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.75, 0.61}, {1.12, 1.00}, {1.95, 1.70}, {1.30, 0.86}, {0.60, 0.11},
+                                                              {0.70, 0.18}};
     static constexpr bool seeded = false;
     RofPar par;
     size_t field_size(int) const { return sizeof(float); }

@@ -227,7 +227,8 @@ struct SbDeep {
     using Args = SbDeepArgs;
     // two sweeps and a forward difference: two columns at low edges, three at high ones
     static constexpr int NF = 5, rlo = 2, rhi = 3, words = 11;
-    static constexpr DeepIterCost cost[kDeepShapeCount] = {{1.0, 0.8}, {1.4, 1.4}, {2.2, 2.2}, {1.5, 1.1}};
+    static constexpr DeepIterCost cost[kDeepShapeCount] = {{1.0, 0.8}, {1.4, 1.4}, {2.2, 2.2}, {1.5, 1.1}, {0.8, 0.2},
+                                                              {0.9, 0.3}};
     static constexpr bool seeded = false;
     SbPar par;
     bool aniso;

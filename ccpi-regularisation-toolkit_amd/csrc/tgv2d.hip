@@ -235,7 +235,8 @@ template <typename S>
 struct TgvDeep {
     using Args = TgvDeepArgs;
     static constexpr int NF = 8, rlo = 1, rhi = 1, words = 17;
-    static constexpr DeepIterCost cost[kDeepShapeCount] = {{1.22, 1.65}, {1.90, 2.20}, {3.50, 4.90}, {2.20, 1.40}};
+    static constexpr DeepIterCost cost[kDeepShapeCount] = {{1.22, 1.65}, {1.90, 2.20}, {3.50, 4.90}, {2.20, 1.40}, {0.90, 0.18},
+                                                              {1.10, 0.30}};
     static constexpr bool seeded = false;
     TgvPar par;
     size_t field_size(int i) const { return i == 0 ? sizeof(float) : sizeof(S); }

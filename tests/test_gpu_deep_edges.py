@@ -59,3 +59,35 @@ def test_dtv_allocates_once(shape):
     finally:
         lib.cilreg_inject_alloc_failure(0)
     _same(got, want, f"{shape}")
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("method", ["fgp", "pd", "tgv", "rof", "sb", "ndf", "dtv"])
+def test_images_of_few_rows(method, rows):
+    """Long images that regions of 4 and 8 rows cover, and one row more: equal
+    to one iteration per launch in every storage type, with and without stops,
+    at widths around one and several regions."""
+    from ccpi.filters import device as D
+
+    def run(x, iters, tol, p, **kw):
+        if method == "fgp":
+            return D.fgp(x, 0.03, iters, tol, 0, 1, precision=p, **kw)
+        if method == "pd":
+            return D.pd(x, 0.03, iters, tol, 8, 1, 1, precision=p, **kw)
+        if method == "tgv":
+            return D.tgv(x, 0.05, 1.3, 1.7, iters, 12.0, tol, precision=p, **kw)
+        if method == "rof":
+            return D.rof(x, 0.04, iters, 0.002, tol, **kw)
+        if method == "sb":
+            return D.sb(x, 0.05, iters, tol, 0, **kw)
+        if method == "ndf":
+            return D.ndf(x, 0.3, 0.2, iters, 0.2, 2, tol, **kw)
+        return D.dtv(x, _vol(tuple(x.shape), 9), 0.03, iters, tol, 0.05, 0, 1, **kw)
+
+    for width in (63, 64, 65, 40011):
+        x = _vol((rows, width), rows)
+        for p in ("fp32", "bf16", "fp16") if method in ("fgp", "pd", "tgv") else ("fp32",):
+            for iters, tol in ((19, 0.0), (25, 2e-2)):
+                kw = {"check_every": 2} if tol else {}
+                _same(run(x, iters, tol, p, depth=1, **kw), run(x, iters, tol, p, **kw),
+                      f"{method} {rows} x {width} {p} tol={tol}")
