@@ -4,12 +4,14 @@
 
 namespace cilreg {
 
-DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[kDeepShapeCount], int words, int most) {
+DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[kDeepShapeCount], int words, int most,
+                   int rows_per_thread) {
     constexpr double kCus = 256, kBytesPerUs = 4.5e6;
     DeepPlan best{};
     double best_us = 1e300;
     for (int s = 0; s < kDeepShapeCount; ++s) {
         const DeepShapeCost& c = kDeepShapes[s];
+        if (c.r > rows_per_thread) continue;
         const int h = 64 * c.nw / c.lx * c.r;
         for (int w = 1; w <= most; ++w) {
             const int lo = rlo * w, hi = rhi * w;

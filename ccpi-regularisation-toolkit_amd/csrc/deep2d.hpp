@@ -212,8 +212,10 @@ struct DeepIterCost { double alone_us, shared_us; };
 
 struct DeepPlan { int shape, width; Deep2D g; };
 // rlo / rhi: columns lost per iteration at a low / high edge; words: read and
-// written per point and pass; most: the largest width allowed.
-DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[kDeepShapeCount], int words, int most);
+// written per point and pass; most: the largest width allowed; rows: the most
+// rows per thread.
+DeepPlan plan_deep(int nx, int ny, int rlo, int rhi, const DeepIterCost (&cost)[kDeepShapeCount], int words, int most,
+                   int rows);
 
 // Calls fn(DeepShape<...>{}) for shape index s.
 template <class Fn>
@@ -240,7 +242,12 @@ struct DeepExtra {
 // ---------------------------------------------------------------------------
 // the solve loop
 // ---------------------------------------------------------------------------
-// M supplies
+// A method's shapes: the most rows per thread on an nx x ny image.
+struct DeepMethod {
+    static int most_rows(int, int) { return 4; }
+};
+
+// M, a DeepMethod, supplies
 //   using Args                       its DeepArgs
 //   static constexpr int NF          state fields per set
 //   static constexpr int rlo, rhi    columns lost per iteration
@@ -266,7 +273,7 @@ int deep_solve(M& m, const T* d_f, T* d_out, int nx, int ny, int iter, T epsil, 
     const bool use_tol = epsil != (T)0;
     int most = opts.depth >= 2 ? 2 : kDeepMax;
     if (most > iter) most = iter;
-    const DeepPlan plan = plan_deep(nx, ny, M::rlo, M::rhi, M::cost, M::words, most);
+    const DeepPlan plan = plan_deep(nx, ny, M::rlo, M::rhi, M::cost, M::words, most, M::most_rows(nx, ny));
     const int width = plan.width;
 
     Arena ar;

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64 * Sh::NW) void fgp_deep_kernel(FgpDeepArgs a) {
 }
 
 template <typename S, bool DIR = false>
-struct FgpDeep {
+struct FgpDeep : DeepMethod {
     using Args = FgpDeepArgs;
     static constexpr int NF = 4, rlo = 1, rhi = 1, words = DIR ? 11 : 9;
     static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.52, 0.42}, {0.70, 0.72}, {1.08, 1.15}, {0.72, 0.50}, {0.50, 0.085},

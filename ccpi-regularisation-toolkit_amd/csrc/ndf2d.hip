@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64 * Sh::NW) void ndf_deep_kernel(NdfDeepArgs a) {
     deep_store_checks<Sh>(red, nchk, a.partials, a.g.nblocks, p.lin);
 }
 
-struct NdfDeep {
+struct NdfDeep : DeepMethod {
     using Args = NdfDeepArgs;
     static constexpr int NF = 1, rlo = 1, rhi = 1, words = 3;
     static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.5, 0.4}, {0.7, 0.65}, {1.1, 1.05}, {0.75, 0.55}, {0.45, 0.115},

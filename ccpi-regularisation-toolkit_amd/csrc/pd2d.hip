@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * Sh::NW) void pd_deep_kernel(PdDeepArgs a) {
 }
 
 template <typename S>
-struct PdDeep {
+struct PdDeep : DeepMethod {
     using Args = PdDeepArgs;
     static constexpr int NF = 3, rlo = 1, rhi = 1, words = 7;
     static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.53, 0.48}, {0.85, 0.82}, {1.40, 1.70}, {0.85, 0.70}, {0.50, 0.09},

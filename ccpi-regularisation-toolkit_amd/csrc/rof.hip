@@ -40,7 +40,7 @@ int rof_solve(const T* d_f, T* d_out, T lambda, int iter, T tau, T epsil, int nx
         CILREG_CK(hipStreamSynchronize(s));
         return 0;
     }
-    if (dim == 2 && opts.depth != 1 && nx > 1 && ny > 1)
+    if (dim == 2 && opts.depth != 1)
         return rof_solve_2d(d_f, d_out, lambda, iter, tau, epsil, nx, ny, opts, s, iters_done, re);
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;

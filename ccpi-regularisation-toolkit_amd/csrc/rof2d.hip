@@ -102,6 +102,7 @@ void rof_deep_kernel(RofDeepArgs a) {
                 deep_keep_branch();
                 ul[r] = xfirst ? q : l;
                 ur[r] = xlast ? l : q;
+                if (R == 1 && p.nx == 1) ul[r] = ur[r] = u[r];   // the mirror of a single column is itself
             }
             const T dn = r + 1 < R ? u[r + 1 < R ? r + 1 : r] : ub, up = r > 0 ? u[r > 0 ? r - 1 : 0] : ua;
             uu[r] = up;
@@ -110,6 +111,7 @@ void rof_deep_kernel(RofDeepArgs a) {
                 deep_keep_branch();
                 uu[r] = p.y + r == 0 ? dn : up;
                 ud[r] = p.y + r == p.ny - 1 ? up : dn;
+                if (R == 1 && p.ny == 1) uu[r] = ud[r] = u[r];
             }
         }
         rof2d_fluxes(u, ul, ur, uu, ud, d1, d2);
@@ -125,11 +127,13 @@ void rof_deep_kernel(RofDeepArgs a) {
             if (p.xedge) {
                 deep_keep_branch();
                 d2m = xfirst ? q : l;
+                if (R == 1 && p.nx == 1) d2m = d2[r];
             }
             T d1m = r > 0 ? d1[r > 0 ? r - 1 : 0] : da;
             if (r == 0 && p.yedge) {
                 deep_keep_branch();
                 d1m = p.y == 0 ? (R > 1 ? d1[R > 1 ? 1 : 0] : db) : d1m;
+                if (R == 1 && p.ny == 1) d1m = d1[0];
             }
             const T dv = (d1[r] - d1m) + (d2[r] - d2m);
             const T un = u[r] + tau * (lam * dv - (u[r] - f[r]));
@@ -155,13 +159,16 @@ void rof_deep_kernel(RofDeepArgs a) {
     deep_store_checks<Sh>(red, nchk, a.partials, a.g.nblocks, p.lin);
 }
 
-struct RofDeep {
+struct RofDeep : DeepMethod {
     using Args = RofDeepArgs;
     // D1, D2 at the low neighbours read u two columns / rows away
     static constexpr int NF = 1, rlo = 2, rhi = 1, words = 3;
     static constexpr DeepIterCost cost[kDeepShapeCount] = {{0.75, 0.61}, {1.12, 1.00}, {1.95, 1.70}, {1.30, 0.86}, {0.60, 0.11},
                                                               {0.70, 0.18}};
     static constexpr bool seeded = false;
+    // a single column or row mirrors onto itself, which only the kernels of one
+    // row per thread provide for (in the others it costs two more spilled registers)
+    static int most_rows(int nx, int ny) { return nx > 1 && ny > 1 ? 4 : 1; }
     RofPar par;
     size_t field_size(int) const { return sizeof(float); }
     void prepare(Args& a, int, int, bool) const { a.par = par; }

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(64 * Sh::NW) void sb_deep_kernel(SbDeepArgs a) {
     deep_store_checks<Sh>(red, nchk, a.partials, a.g.nblocks, p.lin);
 }
 
-struct SbDeep {
+struct SbDeep : DeepMethod {
     using Args = SbDeepArgs;
     // two sweeps and a forward difference: two columns at low edges, three at high ones
     static constexpr int NF = 5, rlo = 2, rhi = 3, words = 11;

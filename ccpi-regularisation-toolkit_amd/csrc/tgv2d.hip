@@ -232,7 +232,7 @@ void tgv_deep_kernel(TgvDeepArgs a) {
 }
 
 template <typename S>
-struct TgvDeep {
+struct TgvDeep : DeepMethod {
     using Args = TgvDeepArgs;
     static constexpr int NF = 8, rlo = 1, rhi = 1, words = 17;
     static constexpr DeepIterCost cost[kDeepShapeCount] = {{1.22, 1.65}, {1.90, 2.20}, {3.50, 4.90}, {2.20, 1.40}, {0.90, 0.18},

@@ -91,3 +91,14 @@ def test_images_of_few_rows(method, rows):
                 kw = {"check_every": 2} if tol else {}
                 _same(run(x, iters, tol, p, depth=1, **kw), run(x, iters, tol, p, **kw),
                       f"{method} {rows} x {width} {p} tol={tol}")
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 2), (2, 1), (1, 40), (1, 63), (1, 500), (31, 1), (33, 1), (64, 1), (65, 1),
+                                   (700, 1), (1, 30011), (30011, 1)], ids=str)
+def test_rof_on_a_single_row_or_column(shape):
+    """The mirrored neighbour of a single column or row is the point itself."""
+    from ccpi.filters import device as D
+    x = _vol(shape, 6)
+    for iters, tol in ((1, 0.0), (8, 0.0), (43, 0.0), (60, 1e-3)):
+        _same(D.rof(x, 0.04, iters, 0.002, tol, depth=1, check_every=3), D.rof(x, 0.04, iters, 0.002, tol, check_every=3),
+              f"{shape} iters={iters} tol={tol}")
