@@ -238,12 +238,33 @@ void deep3_dispatch(int s, Fn&& fn) {
     else fn(DeepShape<64, 8, 2>{});
 }
 
+// What a method's register passes need to be ahead of its passes on 64 x 8
+// tiles beside half a million voxels.
+struct Deep3Least {
+    int rows, planes;   // at least so many
+    bool small;         // also where a small volume's regions cover twice the points of its tiles
+};
 // Volumes the register passes take: enough voxels to fill the chip with
-// regions (below, the two-iteration passes on small tiles do it better: FGP
-// 64^3 5.7 against 6.7 us per iteration, 96^3 11.1 against 9.4) and planes
-// below 2^31 bytes.
-inline bool deep3_fits(int nx, int ny, int nz) {
-    return (size_t)nx * ny * nz >= 500000 && (size_t)nx * ny < ((size_t)1 << 29);
+// regions (FGP 64^3 6.7 us per iteration in registers and 5.7 on tiles, 96^3 9.4
+// and 11.1), planes below 2^31 bytes, and, by method,
+//   rows: a region is 16 or 32 rows high, a tile 8 (2 rows of 5380, 171 planes,
+//     FGP 34 to 50 us and 33 to 40; 5 rows of 2497, 494 planes, 41 and 57),
+//   planes: a chunk repeats T planes at its ends,
+//   small: below 1.2 million voxels regions of 64 x 16 points that lose two
+//     columns and rows a side and are as many as the 64 x 8 tiles (128 x 48 x 128:
+//     12 and 12) step no faster than these (PD 10.6 us and 9.6, FGP 10.4 and 10.3;
+//     of 140 such volumes measured these are the only ones that lose).
+inline bool deep3_fits(int nx, int ny, int nz, const Deep3Least& least) {
+    const size_t sxy = (size_t)nx * ny, n = sxy * nz;
+    if (n < 500000 || sxy >= ((size_t)1 << 29) || ny < least.rows || nz < least.planes) return false;
+    const int tiles = ((nx + 63) / 64) * ((ny + 7) / 8);
+    return least.small || n >= 1200000 || make_deep(nx, ny, 64, 16, 2, 2).nblocks < tiles;
+}
+
+// Rows of whole 128-byte lines whose state (bytes per voxel) streams from HBM:
+// the tiled passes' best case.
+inline bool deep3_lines(int nx, int ny, int nz, size_t bytes) {
+    return nx % 32 == 0 && bytes * nx * ny * nz > kDeep3CacheBytes;
 }
 
 }  // namespace cilreg

@@ -652,8 +652,12 @@ int dtv_solve(const T* d_f, const T* d_ref, T* d_out, T lambda, int iter, T epsi
         // fields stream from HBM in rows of whole 128-byte lines, the tiled
         // pass's best case: 256^3 checked every fifth iteration 157 us tiled and
         // 176 in registers, 190 x 257 x 231 163 and 105, 128^3 25.6 and 22.2.
-        const bool tiled = epsil != (T)0 && nx % 32 == 0 && n * 64 > kDeep3CacheBytes;
-        if (dim == 3 && opts.depth != 1 && deep3_fits(nx, ny, nz) && !tiled)
+        const bool lines = deep3_lines(nx, ny, nz, 64), tiled = epsil != (T)0 && lines;
+        // 2 rows of 5380, 171 planes, 43.6 us in registers, 46.5 on tiles, checked in every iteration 59 and 54; of
+        // 889, 323 planes, 19.7 and 18.6; two planes of 2048 x 2048 98 and 90; 103 x 56 x 125 checked 20.2 and 17.4.
+        const bool every = epsil != (T)0 && opts.check_every == 1;
+        const Deep3Least least{every || n < 1000000 ? 3 : 2, lines ? 3 : 2, epsil == (T)0};
+        if (dim == 3 && opts.depth != 1 && deep3_fits(nx, ny, nz, least) && !tiled)
             return dtv_solve_3d(d_f, refgrad, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, mult, opts, s,
                                 iters_done, re);
     }

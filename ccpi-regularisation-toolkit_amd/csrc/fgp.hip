@@ -87,7 +87,14 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
         // under a scratch limit large images keep the path whose workspace decides what fits
         if (dim == 2 && opts.depth != 1 && !(opts.scratch && (size_t)nx * ny >= kFgp2dPassMaxPixels))
             return fgp_solve_2d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, opts, s, iters_done, re, ws);
-        if (dim == 3 && opts.depth != 1 && !opts.scratch && deep3_fits(nx, ny, nz))
+        // Two planes of 2048 x 2048 79 us in registers, 62 on tiles (3000 x 2500: 96 and 108).  16-bit P: 4 rows of
+        // 2949, 864 planes, bf16 98 and 91, FP16 85 and 89, checked in every iteration 119 and 103, 113 and 102; 6
+        // rows of 2723 36 and 41, checked 40 and 41.
+        constexpr bool narrow = sizeof(S) == 2, bf16 = std::is_same<S, bf16_t>::value;
+        const Deep3Least least{narrow && (bf16 || epsil != 0.0f) ? 5 : 3,
+                               deep3_lines(nx, ny, nz, 12 * sizeof(S) + 4) ? 3 : 2,
+                               !narrow && (size_t)nx * ny >= 64};
+        if (dim == 3 && opts.depth != 1 && !opts.scratch && deep3_fits(nx, ny, nz, least))
             return fgp_solve_3d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, opts, s, iters_done, re,
                                    ws);
     }

@@ -88,7 +88,13 @@ int pd_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, T lipschitz, i
         if (dim == 2 && opts.depth != 1 && nx > 1 && ny > 1)
             return pd_solve_2d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, opts, s, iters_done,
                                   re, ws);
-        if (dim == 3 && opts.depth != 1 && nx > 1 && ny > 1 && deep3_fits(nx, ny, nz))
+        // Two planes of 500 x 1000 9.5 us in registers, 8.5 on tiles, of 2048 x 2048 66 and 50; three 78 and 71, of
+        // 1400 x 1500 37 and 40.  Checked in every iteration four of 2048 x 2048 129 and 112, of 1400 x 1500 67 and
+        // 62; 3 rows of 1407, 1726 planes, 96 and 92.
+        const bool every = epsil != 0.0f && opts.check_every == 1, wide = sizeof(S) == 4;
+        const bool streams = wide && 36 * n > kDeep3CacheBytes, lines = wide && deep3_lines(nx, ny, nz, 36);
+        const Deep3Least least{every ? 4 : 3, every && streams ? 5 : lines ? 4 : 3, false};
+        if (dim == 3 && opts.depth != 1 && nx > 1 && deep3_fits(nx, ny, nz, least))
             return pd_solve_3d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, nz, opts, s,
                                   iters_done, re, ws);
     }

@@ -102,3 +102,26 @@ def test_rof_on_a_single_row_or_column(shape):
     for iters, tol in ((1, 0.0), (8, 0.0), (43, 0.0), (60, 1e-3)):
         _same(D.rof(x, 0.04, iters, 0.002, tol, depth=1, check_every=3), D.rof(x, 0.04, iters, 0.002, tol, check_every=3),
               f"{shape} iters={iters} tol={tol}")
+
+
+@pytest.mark.parametrize("shape", [(140, 2, 2000), (90, 3, 2000), (70, 4, 2000), (60, 5, 1900), (24000, 3, 9), (2, 520, 500),
+                                   (2, 2048, 2048), (3, 420, 410), (3, 1500, 1400), (4, 360, 365), (5, 1120, 1000),
+                                   (103, 56, 125), (128, 48, 128), (256, 8, 512)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("method", ["fgp", "pd", "dtv"])
+def test_volumes_of_few_rows_or_planes(method, shape):
+    """Extents on either side of the lines between the register and the tiled
+    passes: equal to one iteration per launch in every storage type, with and
+    without checks."""
+    from ccpi.filters import device as D
+
+    def run(tol, p, **kw):
+        if method == "dtv":
+            return D.dtv(x, ref, 0.03, 7, tol, 0.05, 0, 1, **kw)
+        return (D.fgp if method == "fgp" else D.pd)(x, 0.03, 7, tol, *((8,) if method == "pd" else ()), 0, 1,
+                                                     precision=p, **kw)
+
+    x, ref = _vol(shape, 2), _vol(shape, 8)
+    for p in ("fp32", "bf16", "fp16") if method != "dtv" else ("fp32",):
+        for tol in (0.0, 1e-9):
+            kw = {"check_every": 2} if tol else {}
+            _same(run(tol, p, depth=1, **kw), run(tol, p, **kw), f"{method} {shape} {p} tol={tol}")
