@@ -68,6 +68,8 @@ int cilreg_fgp_dev_noalloc(const float* d_input, float* d_output, float* infovec
     Opts o = resolve_opts(opts);
     o.autotune = 0;   // timing candidates would allocate
     o.profile = 0;    // per-iteration events would be created
+    const int nz = dimZ <= 1 ? 1 : dimZ;
+    o = tuned_opts(CILREG_FGP, dimX, dimY, nz, methodTV == 0, o);
     hipStream_t s = caller_stream(stream);
     if (!s) { set_error("no stream"); return -1; }
     std::lock_guard<std::mutex> lk(g_scratch_mu[dev]);
@@ -75,7 +77,6 @@ int cilreg_fgp_dev_noalloc(const float* d_input, float* d_output, float* infovec
     if (!p) return -1;
     o.scratch = p;
     o.scratch_bytes = kScratchBytes;
-    const int nz = dimZ <= 1 ? 1 : dimZ;
     int done = 0;
     float re = 0.f;
     int rc;

@@ -19,7 +19,8 @@ struct TuneChoice {
 int autotune(int method, int nx, int ny, int nz, int iso, const Opts& base, bool fixed_ty, TuneChoice* out);
 
 // o with the tuned tiling and depth when o.autotune is set and none of them
-// was given explicitly; o unchanged otherwise (or if tuning fails).
+// was given explicitly; on an image, o with the defaults when it holds
+// autotune's choice for it; o unchanged otherwise (or if tuning fails).
 Opts tuned_opts(int method, int nx, int ny, int nz, int iso, const Opts& o);
 
 }  // namespace cilreg

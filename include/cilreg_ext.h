@@ -244,7 +244,8 @@ CILREG_API int cilreg_tgv_dev_ws(const float *d_input, float *d_output, float *i
  * *ms_per_iter receives its kernel time per iteration.  Cached per process
  * and size class.  method: CILREG_ROF / _FGP / _PD / _TGV; methodTV as for
  * FGP / PD.  The choice never changes results (tiling and depth are
- * bit-neutral). */
+ * bit-neutral).  An image is not timed: its choice is tile_y 4, zchunk 1 and
+ * depth 1 or 2, and a solve given these three runs as with the defaults. */
 CILREG_API int cilreg_autotune(int method, int dimX, int dimY, int dimZ, int methodTV, const cilreg_opts *base,
                                cilreg_opts *best, double *ms_per_iter);
 

@@ -125,3 +125,28 @@ def test_volumes_of_few_rows_or_planes(method, shape):
         for tol in (0.0, 1e-9):
             kw = {"check_every": 2} if tol else {}
             _same(run(tol, p, depth=1, **kw), run(tol, p, **kw), f"{method} {shape} {p} tol={tol}")
+
+
+@pytest.mark.parametrize("method", ["rof", "fgp", "pd", "tgv"])
+def test_applying_an_images_tuned_choice_is_the_default(method):
+    """The options that autotune returns for an image, handed to the solve, give
+    the default's kernels: the fastest pass is as fast (one iteration per launch
+    takes more than twice as long), and the results are the same."""
+    from ccpi.filters import device as D
+    x = _vol((512, 512), 7)
+    c = D.autotune(method, (512, 512))
+
+    def run(**kw):
+        if method == "rof":
+            r = D.rof(x, 0.04, 160, 0.002, profile=True, **kw)
+        elif method == "tgv":
+            r = D.tgv(x, 0.05, 1.3, 1.7, 160, 12.0, profile=True, **kw)
+        else:
+            r = (D.fgp if method == "fgp" else D.pd)(x, 0.03, 160, profile=True, **kw)
+        return r, D.last_profile()[1]
+
+    tuned = {k: c[k] for k in ("tile_y", "zchunk", "depth")}
+    run()
+    (a, ta), (b, tb), (_, t1) = run(), run(**tuned), run(depth=1)
+    _same(a, b, method)
+    assert tb < 0.5 * (ta + t1), f"us per iteration: default {1e3 * ta}, tuned {1e3 * tb}, one per launch {1e3 * t1}"
