@@ -41,6 +41,22 @@ static void launch_fgp(const FgpArgs<T, S>& a, bool iso, bool small, hipStream_t
     }
 }
 
+// Two planes of 2048 x 2048 79 us per iteration in registers, 62 on tiles (3000 x
+// 2500: 96 and 108).  16-bit P: 4 rows of 2949, 864 planes, bf16 98 and 91, FP16
+// 85 and 89, checked in every iteration 119 and 103, 113 and 102; 6 rows of 2723
+// 36 and 41, checked 40 and 41.  Under a scratch limit the tiled passes'
+// workspace decides what fits.
+template <typename S>
+bool fgp_in_registers(int nx, int ny, int nz, float epsil, const Opts& opts) {
+    constexpr bool narrow = sizeof(S) == 2, bf16 = std::is_same<S, bf16_t>::value;
+    const Deep3Least least{narrow && (bf16 || epsil != 0.0f) ? 5 : 3,
+                           deep3_lines(nx, ny, nz, 12 * sizeof(S) + 4) ? 3 : 2, !narrow && (size_t)nx * ny >= 64};
+    return opts.depth != 1 && !opts.scratch && deep3_fits(nx, ny, nz, least);
+}
+template bool fgp_in_registers<float>(int, int, int, float, const Opts&);
+template bool fgp_in_registers<bf16_t>(int, int, int, float, const Opts&);
+template bool fgp_in_registers<_Float16>(int, int, int, float, const Opts&);
+
 // Device-resident FGP solve.  d_out receives D of the final iteration (left
 // untouched when iter == 0); with epsil != 0 its prior contents seed the first
 // residual (FGP_TV_core.c:66,123).
@@ -71,8 +87,7 @@ static void launch_fgp2(const Fgp2Args<T, S>& a, bool iso, bool small, hipStream
 // (fgp2_iter_kernel) unless opts.depth == 1 or, by default, a 2D image has
 // kFgp2dPassMaxPixels or more; an odd last iteration runs on the
 // one-iteration kernel.  2D images in FP32 arithmetic take fgp_solve_2d, volumes
-// deep3_fits accepts fgp_solve_3d (not under a scratch limit, whose workspace is
-// this path's).  P_j lives in buffer
+// that fgp_in_registers accepts fgp_solve_3d.  P_j lives in buffer
 // j mod nbuf (nbuf = 4 with two-iteration passes, which write P_{k+1} and
 // P_{k+2} while reading P_k and P_{k-1}; 3 otherwise).
 template <typename T, typename S>
@@ -87,14 +102,7 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
         // under a scratch limit large images keep the path whose workspace decides what fits
         if (dim == 2 && opts.depth != 1 && !(opts.scratch && (size_t)nx * ny >= kFgp2dPassMaxPixels))
             return fgp_solve_2d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, opts, s, iters_done, re, ws);
-        // Two planes of 2048 x 2048 79 us in registers, 62 on tiles (3000 x 2500: 96 and 108).  16-bit P: 4 rows of
-        // 2949, 864 planes, bf16 98 and 91, FP16 85 and 89, checked in every iteration 119 and 103, 113 and 102; 6
-        // rows of 2723 36 and 41, checked 40 and 41.
-        constexpr bool narrow = sizeof(S) == 2, bf16 = std::is_same<S, bf16_t>::value;
-        const Deep3Least least{narrow && (bf16 || epsil != 0.0f) ? 5 : 3,
-                               deep3_lines(nx, ny, nz, 12 * sizeof(S) + 4) ? 3 : 2,
-                               !narrow && (size_t)nx * ny >= 64};
-        if (dim == 3 && opts.depth != 1 && !opts.scratch && deep3_fits(nx, ny, nz, least))
+        if (dim == 3 && fgp_in_registers<S>(nx, ny, nz, epsil, opts))
             return fgp_solve_3d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, opts, s, iters_done, re,
                                    ws);
     }

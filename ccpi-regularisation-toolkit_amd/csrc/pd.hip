@@ -63,7 +63,23 @@ static void launch_pd2(const Pd2Args<T, S>& a, bool iso, bool small, hipStream_t
     }
 }
 
-// Device-resident PD solve.  Images and (deep3_fits) volumes in FP32 arithmetic
+// Two planes of 500 x 1000 9.5 us per iteration in registers, 8.5 on tiles, of
+// 2048 x 2048 66 and 50; three 78 and 71, of 1400 x 1500 37 and 40.  Checked in
+// every iteration four of 2048 x 2048 129 and 112, of 1400 x 1500 67 and 62; 3
+// rows of 1407, 1726 planes, 96 and 92.
+template <typename S>
+bool pd_in_registers(int nx, int ny, int nz, float epsil, const Opts& opts) {
+    const bool every = epsil != 0.0f && opts.check_every == 1, wide = sizeof(S) == 4;
+    const bool lines = wide && deep3_lines(nx, ny, nz, 36);
+    const bool streams = wide && (size_t)36 * nx * ny * nz > kDeep3CacheBytes;
+    const Deep3Least least{every ? 4 : 3, every && streams ? 5 : lines ? 4 : 3, false};
+    return opts.depth != 1 && nx > 1 && deep3_fits(nx, ny, nz, least);
+}
+template bool pd_in_registers<float>(int, int, int, float, const Opts&);
+template bool pd_in_registers<bf16_t>(int, int, int, float, const Opts&);
+template bool pd_in_registers<_Float16>(int, int, int, float, const Opts&);
+
+// Device-resident PD solve.  Images and (pd_in_registers) volumes in FP32 arithmetic
 // take pd_solve_2d and pd_solve_3d; else, in 3D, iterations run two per pass
 // (pd2_iter_kernel) unless opts.depth == 1; an odd last iteration, and every
 // 2D iteration, runs on the one-iteration kernel.  Each pass reads state set
@@ -88,13 +104,7 @@ int pd_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, T lipschitz, i
         if (dim == 2 && opts.depth != 1 && nx > 1 && ny > 1)
             return pd_solve_2d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, opts, s, iters_done,
                                   re, ws);
-        // Two planes of 500 x 1000 9.5 us in registers, 8.5 on tiles, of 2048 x 2048 66 and 50; three 78 and 71, of
-        // 1400 x 1500 37 and 40.  Checked in every iteration four of 2048 x 2048 129 and 112, of 1400 x 1500 67 and
-        // 62; 3 rows of 1407, 1726 planes, 96 and 92.
-        const bool every = epsil != 0.0f && opts.check_every == 1, wide = sizeof(S) == 4;
-        const bool streams = wide && 36 * n > kDeep3CacheBytes, lines = wide && deep3_lines(nx, ny, nz, 36);
-        const Deep3Least least{every ? 4 : 3, every && streams ? 5 : lines ? 4 : 3, false};
-        if (dim == 3 && opts.depth != 1 && nx > 1 && deep3_fits(nx, ny, nz, least))
+        if (dim == 3 && pd_in_registers<S>(nx, ny, nz, epsil, opts))
             return pd_solve_3d<S>(d_f, d_out, lambda, iter, epsil, lipschitz, method, nonneg, nx, ny, nz, opts, s,
                                   iters_done, re, ws);
     }

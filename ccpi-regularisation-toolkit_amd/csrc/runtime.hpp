@@ -222,7 +222,9 @@ constexpr size_t kFgp2dPassMaxPixels = (size_t)1 << 20;
 constexpr int kGroupZChunk = 32;
 
 // Per-iteration kernel timing of the last profiled solve on this thread.
-struct ProfileStats { double mean_ms = 0, min_ms = 0; int count = 0, passes = 0; };
+// steady_ms: the mean without the first and the last pass (where there are
+// three), which need not read or write the state and may be shorter.
+struct ProfileStats { double mean_ms = 0, min_ms = 0, steady_ms = 0; int count = 0, passes = 0; };
 ProfileStats& thread_profile();
 Opts resolve_opts(const cilreg_opts* o);
 
@@ -342,20 +344,23 @@ int drive_core(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctrl,
         ps = ProfileStats();
         // passes that ran (a stop at iteration j leaves later passes as no-ops)
         const int ran = rc == 0 ? (c.stopped ? c.stop_iter + 1 : iter) : 0;
-        double sum = 0, mn = 1e300;
-        int cnt = 0, its = 0;
+        double sum = 0, mn = 1e300, first = 0, last = 0;
+        int cnt = 0, its = 0, ends = 0;
         for (size_t q = 0; q < pass_k.size(); ++q) {
             if (pass_k[q] >= ran) break;
             float ms = 0.f;
             if (hipEventElapsedTime(&ms, pev[2 * q], pev[2 * q + 1]) == hipSuccess) {
                 sum += ms;
                 its += pass_n[q];
+                if (cnt == 0) { first = ms; ends = pass_n[q]; }
+                last = ms;
                 const double per = ms / pass_n[q];
                 mn = per < mn ? per : mn;
                 ++cnt;
             }
         }
-        if (cnt) { ps.mean_ms = sum / its; ps.min_ms = mn; ps.count = its; ps.passes = cnt; }
+        if (cnt) { ps.mean_ms = ps.steady_ms = sum / its; ps.min_ms = mn; ps.count = its; ps.passes = cnt; }
+        if (cnt >= 3) ps.steady_ms = (sum - first - last) / (its - ends - pass_n[cnt - 1]);
         for (auto& ev2 : pev) if (ev2) (void)hipEventDestroy(ev2);
     }
     if (rc != 0) return rc;

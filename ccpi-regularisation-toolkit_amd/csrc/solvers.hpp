@@ -59,6 +59,12 @@ inline void fgp_multipliers(int iter, const WarmState* ws, std::vector<float>& m
     }
 }
 
+// Whether fgp_solve / pd_solve take a volume to fgp_solve_3d / pd_solve_3d.
+template <typename S>
+bool fgp_in_registers(int nx, int ny, int nz, float epsil, const Opts& opts);
+template <typename S>
+bool pd_in_registers(int nx, int ny, int nz, float epsil, const Opts& opts);
+
 // 2D solves with many iterations per launch (opts.depth: 0 = as many as pay,
 // 2 = two; S: storage of the dual fields).
 template <typename S>

@@ -2,12 +2,15 @@
 // the temporal depth (iterations per pass) of a solve by timing them.
 //
 // For a (method, dual storage, TV type, volume extent) it runs a short
-// fixed-count solve (four iterations) of a synthetic volume of that extent
-// for each candidate -- tile height 8 or 4, z chunk planned by occupancy or
-// 8 / 16 / 32 planes (grouped jobs: the engine's 32-plane chunks after an untimed
-// warm-up solve, eight timed iterations), one or two iterations per pass
-// where the method has both -- takes the per-iteration kernel time from HIP
-// events (the solves' own profiling), and keeps the fastest.  Results are cached per process,
+// fixed-count solve of a synthetic volume of that extent for each candidate --
+// tile height 8 or 4, z chunk planned by occupancy or 8 / 16 / 32 planes (grouped
+// jobs: the engine's 32-plane chunks after an untimed warm-up solve, eight timed
+// iterations), one or two iterations per pass where the method has both (in 3D
+// FGP and PD, two stands for the register passes' own number on volumes they
+// take) -- takes the per-iteration kernel time from HIP events (the solves' own
+// profiling), and keeps the fastest.  A probe has four iterations, or sixteen
+// where a pass may hold four: there the first pass reads no state and the last
+// writes none, so the time is that of the passes between.  Results are cached per process,
 // keyed by the extent rounded up to 64 x 32 x 32, so a batch or a server pays
 // for a size class once.  Every candidate computes the same values bit for bit (the results
 // do not depend on the tiling or the pass width), so tuning never changes an
@@ -20,6 +23,7 @@
 // CU count) and is used only on such a device.
 #include "solvers.hpp"
 #include "tune.hpp"
+#include "deep3d.hpp"
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -202,6 +206,13 @@ TuneChoice image_choice(int method, int nx, int ny) {
     return TuneChoice{4, 1, two ? 2 : 1, 0.0};
 }
 
+template <typename S>
+bool in_registers(int method, int nx, int ny, int nz, const Opts& o) {
+    return method == CILREG_FGP  ? fgp_in_registers<S>(nx, ny, nz, 0.0f, o)
+           : method == CILREG_PD ? pd_in_registers<S>(nx, ny, nz, 0.0f, o)
+                                 : false;
+}
+
 }  // namespace
 
 int autotune(int method, int nx, int ny, int nz, int iso, const Opts& base, bool fixed_ty, TuneChoice* out) {
@@ -264,7 +275,15 @@ int autotune(int method, int nx, int ny, int nz, int iso, const Opts& base, bool
             if (z <= nz) zcs.push_back(z);
     if (zcs.empty()) zcs.push_back(nz);
     TuneChoice best{8, fixed_ty ? zcs.front() : 0, depths.front(), 1e300};
-    const int iters = fixed_ty ? 8 : 4;
+    auto registers = [&](const Opts& o) {
+        if (base.precision == CILREG_BF16) return in_registers<bf16_t>(method, nx, ny, nzp, o);
+        if (base.precision == CILREG_FP16) return in_registers<_Float16>(method, nx, ny, nzp, o);
+        return in_registers<float>(method, nx, ny, nzp, o);
+    };
+    Opts two = base;
+    two.depth = 2;
+    const int iters = fixed_ty ? 8 : registers(two) ? 4 * kDeep3Max : 4;
+    ProfileStats chosen;
     auto run = [&](const Opts& o, int it) {
         if (base.precision == CILREG_BF16) return run_method<bf16_t>(method, in, outv, iso, nx, ny, nzp, it, o, s);
         if (base.precision == CILREG_FP16) return run_method<_Float16>(method, in, outv, iso, nx, ny, nzp, it, o, s);
@@ -279,6 +298,7 @@ int autotune(int method, int nx, int ny, int nz, int iso, const Opts& base, bool
                 o.depth = d;
                 o.autotune = 0;
                 o.profile = 0;
+                if (ty != tys.front() && registers(o)) continue;   // no tiles: timed already
                 // a candidate's first launches run on cold caches and code
                 // objects: an untimed solve first, then the timed one
                 if (fixed_ty && run(o, 2) != 0) return -1;
@@ -286,10 +306,14 @@ int autotune(int method, int nx, int ny, int nz, int iso, const Opts& base, bool
                 const int rc = run(o, iters);
                 if (rc != 0) return -1;
                 const ProfileStats& ps = thread_profile();
-                if (ps.count > 0 && ps.mean_ms < best.ms_per_iter) best = TuneChoice{ty, zc, d, ps.mean_ms};
+                if (ps.count > 0 && ps.steady_ms < best.ms_per_iter) {
+                    best = TuneChoice{ty, zc, d, ps.steady_ms};
+                    chosen = ps;
+                }
             }
         }
     }
+    thread_profile() = chosen;
     std::lock_guard<std::mutex> lk(g_mu);
     g_cache[key] = best;
     *out = best;

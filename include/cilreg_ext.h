@@ -38,7 +38,7 @@ enum { CILREG_FP32 = 0, CILREG_BF16 = 1, CILREG_FP16 = 2 };
 typedef struct cilreg_opts {
     int check_every;     /* residual-check cadence in iterations; 0 = 5 (the reference's) */
     int dual_precision;  /* CILREG_FP32 / CILREG_BF16 / CILREG_FP16 storage of dual and auxiliary fields */
-    int tile_y;          /* tile height in y (4 or 8); 0 = auto */
+    int tile_y;          /* tile height in y (4 or 8; passes in registers have no tiles); 0 = auto */
     int zchunk;          /* z planes marched per workgroup; 0 = auto */
     int profile;         /* 1: time every iteration's kernels with HIP events (see cilreg_last_profile) */
     int wide_index;      /* 1: force 64-bit element indexing (chosen automatically for fields >= 2 GiB) */
@@ -241,10 +241,11 @@ CILREG_API int cilreg_tgv_dev_ws(const float *d_input, float *d_output, float *i
  * given extent for each candidate tiling (tile_y 8/4, zchunk planned or
  * 8/16/32) and temporal depth (1/2 for FGP, PD, TGV in 3D) with base's dual
  * storage, and writes the fastest into *best (base's other fields copied);
- * *ms_per_iter receives its kernel time per iteration.  Cached per process
- * and size class.  method: CILREG_ROF / _FGP / _PD / _TGV; methodTV as for
- * FGP / PD.  The choice never changes results (tiling and depth are
- * bit-neutral).  An image is not timed: its choice is tile_y 4, zchunk 1 and
+ * *ms_per_iter receives its kernel time per iteration in the middle of a solve,
+ * and where it timed anything cilreg_last_profile then describes the probe of
+ * the choice.  Cached per process and size class.  method: CILREG_ROF / _FGP /
+ * _PD / _TGV; methodTV as for FGP / PD.  The choice never changes results
+ * (tiling and depth are bit-neutral).  An image is not timed: its choice is tile_y 4, zchunk 1 and
  * depth 1 or 2, and a solve given these three runs as with the defaults. */
 CILREG_API int cilreg_autotune(int method, int dimX, int dimY, int dimZ, int methodTV, const cilreg_opts *base,
                                cilreg_opts *best, double *ms_per_iter);

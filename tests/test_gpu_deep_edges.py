@@ -150,3 +150,19 @@ def test_applying_an_images_tuned_choice_is_the_default(method):
     (a, ta), (b, tb), (_, t1) = run(), run(**tuned), run(depth=1)
     _same(a, b, method)
     assert tb < 0.5 * (ta + t1), f"us per iteration: default {1e3 * ta}, tuned {1e3 * tb}, one per launch {1e3 * t1}"
+
+
+@pytest.mark.parametrize("method", ["fgp", "pd"])
+def test_tuner_times_the_middle_of_a_register_solve(method):
+    """On a volume the register passes take, a probe holds several of them: four
+    iterations were one pass that read no state and wrote none.  The choice is
+    one of the candidates and leaves the results alone."""
+    from ccpi.filters import device as D
+    shape = (70, 90, 110)
+    D.tune_clear()
+    c = D.autotune(method, shape)
+    assert D.last_profile()[2] == 16
+    assert c["tile_y"] in (4, 8) and c["zchunk"] in (0, 8, 16, 32) and c["depth"] in (1, 2) and c["ms_per_iter"] > 0
+    x = _vol(shape, 3)
+    f = D.fgp if method == "fgp" else D.pd
+    _same(f(x, 0.03, 9, tile_y=c["tile_y"], zchunk=c["zchunk"], depth=c["depth"]), f(x, 0.03, 9), method)
