@@ -152,6 +152,8 @@ int cilreg_last_profile(double* mean_ms, double* min_ms, int* count) {
     return ps.count > 0 ? 0 : -1;
 }
 
+int cilreg_last_profile_passes(void) { return thread_profile().passes; }
+
 int cilreg_release_cache(void) { return pool_release_idle(); }
 
 int cilreg_pool_stats(size_t* busy_bytes, size_t* idle_bytes) {

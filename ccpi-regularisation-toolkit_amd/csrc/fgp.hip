@@ -51,7 +51,7 @@ bool fgp_in_registers(int nx, int ny, int nz, float epsil, const Opts& opts) {
     constexpr bool narrow = sizeof(S) == 2, bf16 = std::is_same<S, bf16_t>::value;
     const Deep3Least least{narrow && (bf16 || epsil != 0.0f) ? 5 : 3,
                            deep3_lines(nx, ny, nz, 12 * sizeof(S) + 4) ? 3 : 2, !narrow && (size_t)nx * ny >= 64};
-    return opts.depth != 1 && !opts.scratch && deep3_fits(nx, ny, nz, least);
+    return opts.depth != 1 && !opts.tiled && !opts.scratch && deep3_fits(nx, ny, nz, least);
 }
 template bool fgp_in_registers<float>(int, int, int, float, const Opts&);
 template bool fgp_in_registers<bf16_t>(int, int, int, float, const Opts&);

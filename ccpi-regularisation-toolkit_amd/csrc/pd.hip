@@ -73,7 +73,7 @@ bool pd_in_registers(int nx, int ny, int nz, float epsil, const Opts& opts) {
     const bool lines = wide && deep3_lines(nx, ny, nz, 36);
     const bool streams = wide && (size_t)36 * nx * ny * nz > kDeep3CacheBytes;
     const Deep3Least least{every ? 4 : 3, every && streams ? 5 : lines ? 4 : 3, false};
-    return opts.depth != 1 && nx > 1 && deep3_fits(nx, ny, nz, least);
+    return opts.depth != 1 && !opts.tiled && nx > 1 && deep3_fits(nx, ny, nz, least);
 }
 template bool pd_in_registers<float>(int, int, int, float, const Opts&);
 template bool pd_in_registers<bf16_t>(int, int, int, float, const Opts&);

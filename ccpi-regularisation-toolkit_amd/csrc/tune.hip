@@ -296,6 +296,7 @@ int autotune(int method, int nx, int ny, int nz, int iso, const Opts& base, bool
                 o.tile_y = ty;
                 o.zchunk = zc;
                 o.depth = d;
+                o.tiled = fixed_ty;
                 o.autotune = 0;
                 o.profile = 0;
                 if (ty != tys.front() && registers(o)) continue;   // no tiles: timed already

@@ -85,6 +85,8 @@ CILREG_API const char *cilreg_last_error(void);
  * launch of the iteration kernel(s) (the stopping-rule finaliser excluded);
  * a launch that advances several iterations counts its time divided by them. */
 CILREG_API int cilreg_last_profile(double *mean_ms, double *min_ms, int *count);
+/* The launches those iterations ran in. */
+CILREG_API int cilreg_last_profile_passes(void);
 
 /* Frees the device memory the library keeps cached between calls on the
  * current device (solves reuse freed workspaces instead of calling hipMalloc;

@@ -166,3 +166,24 @@ def test_tuner_times_the_middle_of_a_register_solve(method):
     x = _vol(shape, 3)
     f = D.fgp if method == "fgp" else D.pd
     _same(f(x, 0.03, 9, tile_y=c["tile_y"], zchunk=c["zchunk"], depth=c["depth"]), f(x, 0.03, 9), method)
+
+
+@pytest.mark.parametrize("method", ["fgp", "pd"])
+def test_tuner_times_a_groups_own_passes(method, tmp_path):
+    """The probe for a grouped job runs the tiled passes that the group runs: two
+    iterations each at depth 2, also where a single solve of the stacked extent
+    would run in registers."""
+    import ctypes
+    from ccpi.filters import batch as B, device as D
+    from ccpi.filters.utils import require_gpu_lib
+    lib = require_gpu_lib()
+    lib.cilreg_last_profile_passes.restype = ctypes.c_int
+    D.tune_clear()
+    x = _vol((40, 70, 100), 1)
+    spec = {"method": method, "input": x, "iters": 6, "lambda": 0.03, "L": 12.0}
+    B.batch_run([spec, dict(spec)], autotune=True)
+    D.tune_save(tmp_path / "t.txt")
+    rows = [l.split() for l in open(tmp_path / "t.txt") if not l.startswith("#")]
+    assert len(rows) == 1 and rows[0][4] == "1"   # the grouped entry
+    depth = int(rows[0][10])
+    assert D.last_profile()[2] == 8 and lib.cilreg_last_profile_passes() == 8 // depth
