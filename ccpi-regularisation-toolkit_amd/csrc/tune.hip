@@ -19,8 +19,8 @@
 // The choices persist in a text file when the caller asks for it
 // (cilreg_tune_save / cilreg_tune_load, or CILREG_TUNE_CACHE=<path>: loaded
 // before the first tuning of the process and rewritten after every new
-// choice).  Each entry names the device it was measured on (architecture and
-// CU count) and is used only on such a device.
+// choice).  Each entry names the device it was measured on (architecture, CU
+// count and the kernels' generation) and is used only on such a device.
 #include "solvers.hpp"
 #include "tune.hpp"
 #include "deep3d.hpp"
@@ -38,7 +38,7 @@ namespace cilreg {
 namespace {
 
 struct Key {
-    std::string device;   // architecture name and CU count, e.g. "gfx950:256"
+    std::string device;   // architecture name, CU count and kernels, e.g. "gfx950:256:k2"
     int method, precision, iso, fixed_ty, nx, ny, nz;
     bool operator<(const Key& o) const {
         return std::tie(device, method, precision, iso, fixed_ty, nx, ny, nz) <
@@ -50,9 +50,14 @@ std::map<Key, TuneChoice> g_cache;
 bool g_env_loaded = false;   // CILREG_TUNE_CACHE read (guarded by g_mu)
 
 constexpr const char* kCacheHeader = "# cilreg autotune cache v1";
+// Raised when a method's kernels change so that choices timed on the ones
+// before no longer hold: such entries are kept and saved, but not used.  (1: no
+// suffix, two-iteration tiled passes; k2: register passes -- a depth of 1 would
+// turn them off, chunks of 8 planes would have them march twice the planes.)
+constexpr const char* kKernels = "k2";
 
 // Identity of the current device for the cache: its architecture (the first
-// field of gcnArchName) and its CU count; looked up once per device.
+// field of gcnArchName), its CU count and kKernels; looked up once per device.
 int device_identity(std::string* id) {
     static std::mutex mu;
     static std::map<int, std::string> known;
@@ -78,7 +83,7 @@ int device_identity(std::string* id) {
     if (arch.empty()) arch = "unknown";
     for (char& ch : arch)
         if (ch == ' ') ch = '_';   // one whitespace-free field of the file
-    *id = known[dev] = arch + ":" + std::to_string(prop.multiProcessorCount);
+    *id = known[dev] = arch + ":" + std::to_string(prop.multiProcessorCount) + ":" + kKernels;
     return 0;
 }
 

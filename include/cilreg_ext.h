@@ -256,8 +256,9 @@ CILREG_API int cilreg_autotune(int method, int dimX, int dimY, int dimZ, int met
  * whose tile sizes are compile-time constants).  First line
  * "# cilreg autotune cache v1", then one entry per line:
  *   device method precision iso grouped nx ny nz tile_y zchunk depth ms_per_iter
- * device = architecture and CU count ("gfx950:256"); an entry is used only on
- * such a device.  cilreg_tune_save writes every cached choice (through
+ * device = architecture, CU count and the generation of the kernels the choice
+ * was timed on ("gfx950:256:k2"); an entry is used only on such a device and by
+ * such kernels.  cilreg_tune_save writes every cached choice (through
  * path.tmp and a rename) and returns the number written; cilreg_tune_load
  * merges a file into the process's cache (replacing entries with the same
  * key) and returns the number read -- a file with a malformed line is

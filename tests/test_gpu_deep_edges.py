@@ -187,3 +187,25 @@ def test_tuner_times_a_groups_own_passes(method, tmp_path):
     assert len(rows) == 1 and rows[0][4] == "1"   # the grouped entry
     depth = int(rows[0][10])
     assert D.last_profile()[2] == 8 and lib.cilreg_last_profile_passes() == 8 // depth
+
+
+def test_choices_timed_on_earlier_kernels_are_not_used(tmp_path):
+    """An entry for this device without the kernels' generation was timed before
+    the register passes: it loads and saves, and the tuner times anew."""
+    from ccpi.filters import device as D
+    shape = (70, 90, 110)
+    D.tune_clear()
+    D.autotune("fgp", shape)
+    D.tune_save(tmp_path / "new.txt")
+    header, row = [l for l in open(tmp_path / "new.txt") if not l.startswith("# device")]
+    f = row.split()
+    assert f[0].count(":") == 2
+    f[0] = f[0].rsplit(":", 1)[0]
+    f[8:11] = ["4", "8", "1"]
+    f[11] = "123.0"
+    (tmp_path / "old.txt").write_text(header + " ".join(f) + "\n")
+    D.tune_clear()
+    assert D.tune_load(tmp_path / "old.txt") == 1
+    assert D.autotune("fgp", shape)["ms_per_iter"] != 123.0
+    assert D.tune_entries() == 2   # the old entry is still there to save
+    D.tune_clear()
