@@ -99,8 +99,10 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
     *re = 0.f;
     if (iter <= 0) return 0;
     if constexpr (std::is_same<T, float>::value) {
-        // under a scratch limit large images keep the path whose workspace decides what fits
-        if (dim == 2 && opts.depth != 1 && !(opts.scratch && (size_t)nx * ny >= kFgp2dPassMaxPixels))
+        // Under a scratch limit large images keep the path whose workspace decides what fits, unless two iterations
+        // per launch are asked for: eight or nine fields, where two-iteration tiled passes had ten.
+        if (dim == 2 && opts.depth != 1 &&
+            !(opts.scratch && !(opts.depth == 2 && iter > 1) && (size_t)nx * ny >= kFgp2dPassMaxPixels))
             return fgp_solve_2d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, opts, s, iters_done, re, ws);
         if (dim == 3 && fgp_in_registers<S>(nx, ny, nz, epsil, opts))
             return fgp_solve_3d<S>(d_f, d_out, lambda, iter, epsil, method, nonneg, nx, ny, nz, opts, s, iters_done, re,
@@ -110,10 +112,11 @@ int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, i
     const bool small = !opts.wide_index && fits_u32(n, sizeof(T) > sizeof(S) ? sizeof(T) : sizeof(S));
     const int ty = (opts.tile_y == 4 || dim == 2) ? 4 : 8;
     const bool iso = method == 0;
-    // returning the state after a stop needs the stop iteration's own pass
+    // returning the state after a stop needs the stop iteration's own pass; FP32 images come here for one
+    // iteration per launch only
     const bool pass2 = opts.depth == 2 || (opts.depth == 0 && (dim == 3 || n < kFgp2dPassMaxPixels));
-    const bool two = pass2 && iter > 1 && !(ws && epsil != (T)0);
-    const int width = (two && (dim == 3 || std::is_same<T, double>::value)) ? 2 : 1;
+    const bool two = pass2 && iter > 1 && !(ws && epsil != (T)0) && (dim == 3 || std::is_same<T, double>::value);
+    const int width = two ? 2 : 1;
     // 2D two-iteration passes: 64 x 4 tiles unless 8 rows are asked for
     const int ty2d = opts.tile_y == 8 ? 8 : 4;
     Geom g;

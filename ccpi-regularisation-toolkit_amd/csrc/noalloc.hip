@@ -3,8 +3,9 @@
 // cilreg_fgp_dev_noalloc is cilreg_fgp_dev for callers that cannot allocate
 // device memory (code that must not call hipMalloc, tight serving loops,
 // harnesses that forbid it): the solve's workspace -- the dual fields P (three
-// or four sets), the two objective buffers D, the stopping-rule control block
-// and the per-workgroup residual partials -- is carved from `scratch`, a
+// or four sets) and the two objective buffers D, or, for images that run in
+// registers, two sets of state, the stopping-rule control block and the
+// per-workgroup residual partials -- is carved from `scratch`, a
 // file-scope device array of kScratchBytes, instead of the library's pool.
 // Each GPU the library runs on holds its own copy of the array from the
 // moment the code object is loaded until the process ends.

@@ -152,8 +152,8 @@ CILREG_API int cilreg_dtv_dev(const float *d_input, const float *d_ref, float *d
  * reference: for callers that cannot allocate device memory (code that must
  * not call hipMalloc, serving loops, harnesses that forbid it).  Volumes
  * whose workspace exceeds the array (FP32 3D: 56 B per voxel, about 1.19 M
- * voxels; 2D: 40 B per pixel; BF16/FP16 duals: 32 and 24 B) return -1 with
- * that reason.  Calls on one device share the array and are serialised by
+ * voxels; 2D: 32 B per pixel, 36 in place; BF16/FP16 duals: 32 and 20 B) return
+ * -1 with that reason.  Calls on one device share the array and are serialised by
  * the library; the array keeps the last call's contents. */
 CILREG_API int cilreg_fgp_dev_noalloc(const float *d_input, float *d_output, float *infovector, float lambdaPar,
                                       int iter, float epsil, int methodTV, int nonneg, int dimX, int dimY, int dimZ,

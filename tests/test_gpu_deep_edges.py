@@ -209,3 +209,28 @@ def test_choices_timed_on_earlier_kernels_are_not_used(tmp_path):
     assert D.autotune("fgp", shape)["ms_per_iter"] != 123.0
     assert D.tune_entries() == 2   # the old entry is still there to save
     D.tune_clear()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("shape, in_place", [((1100, 1000), True), ((1300, 1380), True), ((1401, 1301), False)], ids=str)
+def test_allocation_free_large_image_two_iterations_per_launch(shape, in_place, precision):
+    """depth=2 on an image of 2^20 pixels and more: two iterations per launch in a
+    workspace of eight fields (nine in place); ten were reserved for passes of
+    one iteration, which left no room from 1.68 million pixels on."""
+    import ctypes
+    import torch
+    from ccpi.filters import device as D
+    from ccpi.filters.utils import last_error, require_gpu_lib
+    f = require_gpu_lib().cilreg_fgp_dev_noalloc
+    vp, i, fl = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    f.argtypes, f.restype = [vp, vp, vp, fl, i, fl, i, i, i, i, i, vp, vp], i
+    for iters in (1, 2, 7):
+        x = _vol(shape, 5)
+        want = D.fgp(x, 0.03, iters, 0.0, 0, 1, precision=precision, depth=1)
+        out = x if in_place else torch.zeros_like(x)
+        info = np.zeros(2, dtype=np.float32)
+        opts = D.make_opts(precision=precision, depth=2)
+        rc = f(x.data_ptr(), out.data_ptr(), info.ctypes.data, 0.03, iters, 0.0, 0, 1, shape[1], shape[0], 1,
+               ctypes.byref(opts), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, last_error()
+        _same((out, info), want, f"{shape} iters={iters}")
