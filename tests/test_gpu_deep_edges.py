@@ -234,3 +234,57 @@ def test_allocation_free_large_image_two_iterations_per_launch(shape, in_place, 
                ctypes.byref(opts), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
         assert rc == 0, last_error()
         _same((out, info), want, f"{shape} iters={iters}")
+
+
+def _same64(a, b, tag):
+    import torch
+    assert np.array_equal(a[1], b[1]), f"{tag}: infovector {a[1]} vs {b[1]}"
+    assert bool((a[0].view(torch.int64) == b[0].view(torch.int64)).all()), tag
+
+
+@pytest.mark.parametrize("wide_index", [False, True])
+@pytest.mark.parametrize("tile_y", [4, 8])
+def test_fp64_images_two_iterations_per_pass(tile_y, wide_index):
+    """The two-iteration tiled pass of an image, which only FP64 still takes:
+    equal to one iteration per launch on both tile heights with either index
+    width, for odd and even counts and stops on either iteration of a pass."""
+    from ccpi.filters import device as D
+    kw = dict(tile_y=tile_y, wide_index=wide_index)
+    for shape in ((5, 7), (33, 64), (63, 65), (130, 201)):
+        x = _vol(shape, 3).double()
+        for iters, aniso in ((1, 0), (2, 1), (9, 0), (10, 1)):
+            _same64(D.fgp_f64(x, 0.03, iters, 0.0, aniso, 1, depth=1, **kw),
+                    D.fgp_f64(x, 0.03, iters, 0.0, aniso, 1, depth=2, **kw), f"{shape} iters={iters}")
+    stops = set()
+    x = _vol((120, 140), 5).double()
+    for check_every in (1, 2, 3):
+        for tol in (3e-2, 2e-2, 1e-2, 5e-3, 3e-3):
+            a = D.fgp_f64(x, 0.03, 90, tol, 0, 1, depth=1, check_every=check_every, **kw)
+            _same64(a, D.fgp_f64(x, 0.03, 90, tol, 0, 1, depth=2, check_every=check_every, **kw),
+                    f"tol={tol} check_every={check_every}")
+            stops.add(int(a[1][0]))
+    assert {k & 1 for k in stops if k < 90} == {0, 1}
+
+
+@pytest.mark.parametrize("method", ["rof", "fgp", "pd", "tgv", "dtv", "sb", "ndf"])
+def test_one_iteration_kernels_of_images_with_64_bit_indexes(method):
+    """depth=1 keeps the one-iteration kernels; both index widths agree."""
+    from ccpi.filters import device as D
+    x, ref = _vol((101, 133), 3), _vol((101, 133), 4)
+
+    def run(**kw):
+        if method == "rof":
+            return D.rof(x, 0.04, 13, 0.002, 1e-9, depth=1, **kw)
+        if method == "fgp":
+            return D.fgp(x, 0.03, 13, 1e-9, 0, 1, depth=1, **kw)
+        if method == "pd":
+            return D.pd(x, 0.03, 13, 1e-9, 12.0, 0, 1, depth=1, **kw)
+        if method == "tgv":
+            return D.tgv(x, 0.05, 1.3, 1.7, 13, 12.0, 1e-9, depth=1, **kw)
+        if method == "dtv":
+            return D.dtv(x, ref, 0.03, 13, 1e-9, 0.05, 0, 1, depth=1, **kw)
+        if method == "sb":
+            return D.sb(x, 0.05, 13, 1e-9, 0, depth=1, **kw)
+        return D.ndf(x, 0.3, 0.2, 13, 0.2, 2, 1e-9, depth=1, **kw)
+
+    _same(run(), run(wide_index=True), method)
