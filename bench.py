@@ -8,10 +8,10 @@ checked every iteration.  One step = one full solve with the input already in
 HBM; value = voxel-iterations per second over the timed steps.
 
 Also reported:
-* roofline: the FGP kernel's algorithmic bytes (48 B per voxel-iteration with
-  the every-iteration residual check; a launch advances two iterations) over
-  its launch time, measured with HIP events on the solve's stream around every
-  launch;
+* roofline: the bytes that a launch of the FGP kernel cannot do without (60 B
+  per voxel with the every-iteration residual check, for as many iterations as
+  the launch advances) over its launch time, measured with HIP events on the
+  solve's stream around every launch;
 * cpu_baseline: the reference C-OMP library (oracle/_ref, built from the
   reference sources) or, where it is absent, the C restatement (oracle/), on a
   bounded sample of the same workload, on the host's cores; with the extras,
@@ -70,6 +70,47 @@ def run_fgp(D, x, profile=False):
     p = FGP_PARAMS
     return D.fgp(x, p["lam"], p["iters"], p["tol"], p["method"], p["nonneg"], check_every=p["check_every"],
                  profile=profile)
+
+
+# Bytes per voxel that a launch reads and writes once, however many iterations
+# it advances.  FGP: f, P_k and P_{k-1} (3 components each) and, checked, the
+# objective D of the iteration before; P and P_{k-1} again and D.  PD: u_bar, f,
+# P; u_bar, P.  FGP-dTV: as FGP without D, and B.  SB: U, f, D, B; U, D, B.  TGV:
+# u_bar, f, v_bar, P, Q; all but f.  Diffusion: u, f; u.
+LAUNCH_BYTES = {"fgp_checked": 60, "pd": 36, "pd_16bit": 24, "dtv": 64, "sb": 60, "tgv": 108, "tgv_16bit": 60,
+                "diffusion": 12}
+
+
+def launch_rate(n_voxels, kind, mean_ms, count, passes):
+    """What a profiled solve says of its kernel: time per iteration and per
+    launch, and the rate of the bytes a launch cannot do without."""
+    if not (mean_ms and count and passes):
+        return {"kernel_ms_mean": None, "kernel_alg_GBps": None}
+    per_launch = count / passes
+    gbps = LAUNCH_BYTES[kind] * n_voxels / (mean_ms * per_launch * 1e-3) / 1e9
+    return {"kernel_ms_mean": mean_ms, "iterations_timed": count, "iterations_per_launch": per_launch,
+            "launch_ms_mean": mean_ms * per_launch, "alg_bytes_per_voxel_launch": LAUNCH_BYTES[kind],
+            "kernel_alg_GBps": gbps, "kernel_frac_of_8TBps": gbps / HBM_PEAK_GBS}
+
+
+def profiled_rate(D, n_voxels, kind):
+    from ccpi.filters.utils import require_gpu_lib
+    mean_ms, _, count = D.last_profile()
+    return launch_rate(n_voxels, kind, mean_ms, count, require_gpu_lib().cilreg_last_profile_passes())
+
+
+def roofline_of(n_voxels, mean_ms, min_ms, count, passes, traffic, achievable):
+    """The headline kernel against the HBM peak, from a profiled checked solve."""
+    r = launch_rate(n_voxels, "fgp_checked", mean_ms, count, passes)
+    achieved = r["kernel_alg_GBps"]
+    per_launch = r.get("iterations_per_launch")
+    return {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
+            "kernel": "fgp_deep3_kernel", "iterations_per_launch": per_launch,
+            "kernel_ms_mean": r.get("launch_ms_mean"), "kernel_ms_min": min_ms * per_launch if per_launch else None,
+            "kernel_ms_mean_per_iteration": mean_ms, "iterations_timed": count,
+            "alg_bytes_per_launch": LAUNCH_BYTES["fgp_checked"] * n_voxels, "achievable_GBps": achievable,
+            "frac_of_achievable_sum2": achieved / achievable["sum2"] if achieved else None}
 
 
 def read_traffic(n_voxels):
@@ -194,11 +235,9 @@ def secondary(D, torch):
         torch.cuda.synchronize()
         dt = time.perf_counter() - t0
         D.tgv(x, *tgv_args, 50, 12.0, 0.0, precision=prec, profile=True)
-        m, _, _ = D.last_profile()
-        b = 108 if prec == "fp32" else 60
         results[prec] = {"y": y, "voxel_iters_per_s": n * info[0] / dt, "seconds": round(dt, 4),
-                         "iterations": int(info[0]), "kernel_ms_mean": m, "alg_bytes_per_voxel_iter": b,
-                         "kernel_alg_GBps": b * n / (m * 1e-3) / 1e9 if m else None}
+                         "iterations": int(info[0]),
+                         **profiled_rate(D, n, "tgv" if prec == "fp32" else "tgv_16bit")}
     log("bench: TGV FP64 reference solve")
     x64 = x.double()
     torch.cuda.synchronize()
@@ -214,8 +253,6 @@ def secondary(D, torch):
         r["objective_fp64"] = objective(y)
         out[f"tgv_3d_192x512x512_{prec}"] = r
     out["tgv_3d_192x512x512_fp64_reference"] = {"seconds": round(t64, 4), "objective_fp64": objective(ref)}
-    out["tgv_3d_192x512x512_fp32"]["kernel_frac_of_8TBps"] = (
-        out["tgv_3d_192x512x512_fp32"]["kernel_alg_GBps"] / HBM_PEAK_GBS)
     del ref, x
     # PD 3D
     log("bench: PD-TV 3D 256^3")
@@ -228,11 +265,9 @@ def secondary(D, torch):
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
     D.pd(x, 0.02, 50, 0.0, 12.0, 0, 1, profile=True)
-    m, _, _ = D.last_profile()
     out["pd_tv_3d_256_fp32"] = {
         "voxel_iters_per_s": n * info[0] / dt, "iterations": int(info[0]), "seconds": round(dt, 4),
-        "kernel_ms_mean": m, "alg_bytes_per_voxel_iter": 36,
-        "kernel_alg_GBps": 36 * n / (m * 1e-3) / 1e9 if m else None}
+        "kernel": "pd_deep3_kernel", **profiled_rate(D, n, "pd")}
     # PD precision study: P stored in FP32 / BF16 / FP16 against an FP64 solve (400 iterations, no tolerance)
     log("bench: PD-TV 3D 256^3 precision study")
     ref, _ = D.pd_f64(x.double(), 0.02, 400, 0.0, 12.0, 0, 1)
@@ -244,12 +279,9 @@ def secondary(D, torch):
         torch.cuda.synchronize()
         dtp = time.perf_counter() - t0
         D.pd(x, 0.02, 50, 0.0, 12.0, 0, 1, precision=prec, profile=True)
-        mp, _, _ = D.last_profile()
-        b = 36 if prec == "fp32" else 24   # P at 2 B: read u_bar, f (8) + P (6); write u_bar (4) + P (6)
         out[f"pd_tv_3d_256_{prec}_duals"] = {
             "voxel_iters_per_s": n * info[0] / dtp, "iterations": int(info[0]), "seconds": round(dtp, 4),
-            "kernel_ms_mean": mp, "alg_bytes_per_voxel_iter": b,
-            "kernel_alg_GBps": b * n / (mp * 1e-3) / 1e9 if mp else None,
+            **profiled_rate(D, n, "pd" if prec == "fp32" else "pd_16bit"),
             "rel_l2_vs_fp64": float(torch.linalg.vector_norm(y.double() - ref)) / ref_norm}
         del y
     del ref
@@ -262,11 +294,9 @@ def secondary(D, torch):
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
     D.sb(x, 0.02, 30, 0.0, 0, profile=True)
-    m, _, _ = D.last_profile()
     out["sb_tv_3d_256_fp32"] = {
         "voxel_iters_per_s": n * info[0] / dt, "iterations": int(info[0]), "seconds": round(dt, 4),
-        "kernel": "sb_fused_kernel<3,8,float,iso,uint32>", "kernel_ms_mean": m, "alg_bytes_per_voxel_iter": 60,
-        "kernel_alg_GBps": 60 * n / (m * 1e-3) / 1e9 if m else None}
+        "kernel": "sb_fused_kernel<3,8,float,iso,uint32>", **profiled_rate(D, n, "sb")}
     # FGP-dTV 3D, guided by the clean phantom with 1% noise
     log("bench: FGP-dTV 3D 256^3")
     out["fgp_dtv_3d_256_fp32"] = dtv_section(D, torch, x)
@@ -304,13 +334,9 @@ def dtv_section(D, torch, x):
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
     D.dtv(x, r, 0.02, 50, 0.0, 0.01, 0, 1, profile=True)
-    m, _, c = D.last_profile()
     return {"voxel_iters_per_s": n * info[0] / dt, "iterations": int(info[0]), "seconds": round(dt, 4),
-            "kernel": "dtv2_iter_kernel<8,float,iso,uint32> (two iterations per launch)", "kernel_ms_mean": m,
-            "iterations_timed": c,
-            "alg_bytes_per_voxel_iter": 52,
-            "kernel_alg_GBps": 52 * n / (m * 1e-3) / 1e9 if m else None,
-            "kernel_frac_of_8TBps": 52 * n / (m * 1e-3) / 1e9 / HBM_PEAK_GBS if m else None}
+            "kernel": "fgp_deep3_kernel (with B; the solve checked every iteration runs dtv2_iter_kernel)",
+            **profiled_rate(D, n, "dtv")}
 
 
 DIFFUSION = {   # the reference tests' parameters (test_2d_cpu_vs_gpu.py:370-377, :431-438, :496-502)
@@ -343,11 +369,9 @@ def diffusion_section(D, torch, x):
         torch.cuda.synchronize()
         dt = time.perf_counter() - t0
         run_diffusion(D, name, x, 50, profile=True)
-        m, _, c = D.last_profile()
         out[f"{name}_3d_256_fp32"] = {
             "voxel_iters_per_s": n * info[0] / dt, "iterations": int(info[0]), "seconds": round(dt, 4),
-            "kernel": DIFFUSION[name][2], "kernel_ms_mean": m, "iterations_timed": c,
-            "alg_bytes_per_voxel_iter": 12, "kernel_alg_GBps": 12 * n / (m * 1e-3) / 1e9 if m else None}
+            "kernel": DIFFUSION[name][2], **profiled_rate(D, n, "diffusion")}
     return out
 
 
@@ -558,9 +582,7 @@ def single_workload(name, steps, D, torch):
     if name == "sb3d":
         x = torch.from_numpy(fgp_workload()).cuda()
         D.sb(x, 0.02, steps, 0.0, 0, profile=True)
-        m, _, c = D.last_profile()
-        return {"workload": "SB-TV 3D 256^3", "kernel_ms_mean_per_iteration": m, "iterations_timed": c,
-                "kernel_alg_GBps": 60 * x.numel() / (m * 1e-3) / 1e9 if m else None}
+        return {"workload": "SB-TV 3D 256^3", **profiled_rate(D, x.numel(), "sb")}
     if name in ("llt3d", "ndf3d", "d43d"):
         x = torch.from_numpy(fgp_workload()).cuda()
         run_diffusion(D, name[:-2], x, steps, profile=True)
@@ -571,9 +593,7 @@ def single_workload(name, steps, D, torch):
         x = torch.from_numpy(fgp_workload()).cuda()
         r = torch.from_numpy(dtv_reference()).cuda()
         D.dtv(x, r, 0.02, steps, 0.0, 0.01, 0, 1, profile=True)
-        m, _, c = D.last_profile()
-        return {"workload": "FGP-dTV 3D 256^3", "kernel_ms_mean_per_iteration": m, "iterations_timed": c,
-                "kernel_alg_GBps": 52 * x.numel() / (m * 1e-3) / 1e9 if m else None}
+        return {"workload": "FGP-dTV 3D 256^3", **profiled_rate(D, x.numel(), "dtv")}
     raise SystemExit(f"unknown workload {name}")
 
 
@@ -645,21 +665,11 @@ def main():
 
     # per-kernel timing with HIP events on the solve's stream
     run_fgp(D, x, profile=True)
-    mean_ms, min_ms, cnt = D.last_profile()   # per iteration (launch time / 2)
-    per_launch = 2
-    bytes_per_launch = 48 * n * per_launch
-    launch_ms = mean_ms * per_launch if mean_ms else None
-    achieved = bytes_per_launch / (launch_ms * 1e-3) / 1e9 if mean_ms else None
-    traffic = read_traffic(n)
-    achievable = D.stream_bench(1 << 30, 20)
-    roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
-                "kernel": "fgp2_iter_kernel<8,float,float,iso,uint32>", "iterations_per_launch": per_launch,
-                "kernel_ms_mean": launch_ms, "kernel_ms_min": min_ms * per_launch if min_ms else None,
-                "kernel_ms_mean_per_iteration": mean_ms, "iterations_timed": cnt,
-                "alg_bytes_per_voxel_iteration": 48, "alg_bytes_per_launch": bytes_per_launch,
-                "achievable_GBps": achievable,
-                "frac_of_achievable_sum2": achieved / achievable["sum2"] if achieved else None}
+    from ccpi.filters.utils import require_gpu_lib
+    mean_ms, min_ms, cnt = D.last_profile()   # per iteration
+    roofline = roofline_of(n, mean_ms, min_ms, cnt, require_gpu_lib().cilreg_last_profile_passes(), read_traffic(n),
+                           D.stream_bench(1 << 30, 20))
+    achieved = roofline["achieved"]
 
     # the same solve through the reference C-ABI on host buffers (PCIe copies
     # included; the reference's every-5 check cadence)
