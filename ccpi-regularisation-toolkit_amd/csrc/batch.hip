@@ -289,8 +289,13 @@ __device__ __attribute__((always_inline)) inline void rof_group_item(const RofJo
     for_tiles<DIM, TY>(a.g, j->h, local, [&](const TileCoord& tc) { rof_body<DIM, TY, T, I>(a, tc); });
 }
 
+// 56 registers (the attribute counts half of the unified file; two spilled, 60
+// without): beside a workgroup of the FGP group,
+// which holds 160 of a SIMD's 512, three of ROF's fit instead of two.  64 volumes,
+// half FGP, half ROF, in one batch: 2.115 -> 2.013 s (16-bit P 1.982 -> 1.878);
+// ROF's half alone 1.266 -> 1.259.
 template <int DIM, int TY, typename T, typename I>
-__global__ __launch_bounds__(TX * TY) void rof_group_kernel(const RofJob<T>* jobs, int njobs, int total, int level) {
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_num_vgpr(28))) void rof_group_kernel(const RofJob<T>* jobs, int njobs, int total, int level) {
     rof_group_item<DIM, TY, T, I>(jobs, njobs, xcd_logical_block((int)blockIdx.x, total), level);
 }
 
