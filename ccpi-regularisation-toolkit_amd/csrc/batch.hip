@@ -494,7 +494,8 @@ __device__ __attribute__((always_inline)) inline void tgv_group_item(const TgvJo
 }
 
 template <int DIM, int TY, typename T, typename S, typename I>
-__global__ __launch_bounds__(TX * TY) void tgv_group_kernel(const TgvJob<T, S>* jobs, int njobs, int total, int level) {
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(tgv_min_waves<DIM, S, I>())))
+void tgv_group_kernel(const TgvJob<T, S>* jobs, int njobs, int total, int level) {
     tgv_group_item<DIM, TY, T, S, I>(jobs, njobs, xcd_logical_block((int)blockIdx.x, total), level);
 }
 

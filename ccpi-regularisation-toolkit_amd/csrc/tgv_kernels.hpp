@@ -395,9 +395,14 @@ __device__ inline void tgv_body(const TgvArgs<T, S>& a, const TileCoord& tc) {
     }
 }
 
+// 3D with 16-bit storage and 64-bit indexes: 128 registers, two 512-thread
+// workgroups per CU (129 and one without the cap: 256^3 280 and 403 us).
+template <int DIM, typename S, typename I>
+constexpr int tgv_min_waves() { return DIM == 3 && sizeof(S) == 2 && sizeof(I) == 8 ? 4 : 1; }
 // One iteration on one volume: the workgroup's tile comes from its block index.
 template <int DIM, int TY, typename T, typename S, typename I>
-__global__ __launch_bounds__(TX * TY) void tgv_iter_kernel(TgvArgs<T, S> a) {
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(tgv_min_waves<DIM, S, I>())))
+void tgv_iter_kernel(TgvArgs<T, S> a) {
     if (solve_stopped(a.ctrl)) return;
     tgv_body<DIM, TY, T, S, I>(a, tile_of_block(a.g, TY));
 }

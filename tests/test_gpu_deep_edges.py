@@ -288,3 +288,14 @@ def test_one_iteration_kernels_of_images_with_64_bit_indexes(method):
         return D.ndf(x, 0.3, 0.2, 13, 0.2, 2, 1e-9, depth=1, **kw)
 
     _same(run(), run(wide_index=True), method)
+
+
+@pytest.mark.parametrize("precision", ["bf16", "fp16"])
+def test_tgv_16bit_one_iteration_kernel_with_64_bit_indexes(precision):
+    from ccpi.filters import batch as B, device as D
+    x = _vol((13, 37, 70), 3)
+    want = D.tgv(x, 0.05, 1.3, 1.7, 9, 12.0, 1e-9, precision=precision, depth=1)
+    _same(want, D.tgv(x, 0.05, 1.3, 1.7, 9, 12.0, 1e-9, precision=precision, depth=1, wide_index=True), precision)
+    spec = {"method": "tgv", "input": x, "iters": 9, "lambda": 0.05, "alpha1": 1.3, "alpha0": 1.7, "L2": 12.0}
+    (y, _), = B.batch_run([spec], precision=precision, depth=1, wide_index=True)
+    assert bool((y == want[0]).all())
