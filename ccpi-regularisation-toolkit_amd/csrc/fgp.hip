@@ -83,13 +83,13 @@ static void launch_fgp2(const Fgp2Args<T, S>& a, bool iso, bool small, hipStream
 
 // Device-resident FGP solve.  d_out receives D of the final iteration (left
 // untouched when iter == 0); with epsil != 0 its prior contents seed the first
-// residual (FGP_TV_core.c:66,123).  Iterations run two per pass
-// (fgp2_iter_kernel) unless opts.depth == 1 or, by default, a 2D image has
-// kFgp2dPassMaxPixels or more; an odd last iteration runs on the
-// one-iteration kernel.  2D images in FP32 arithmetic take fgp_solve_2d, volumes
-// that fgp_in_registers accepts fgp_solve_3d.  P_j lives in buffer
-// j mod nbuf (nbuf = 4 with two-iteration passes, which write P_{k+1} and
-// P_{k+2} while reading P_k and P_{k-1}; 3 otherwise).
+// residual (FGP_TV_core.c:66,123).  In FP32 arithmetic images run on
+// fgp_solve_2d and volumes that fgp_in_registers accepts on fgp_solve_3d.  The
+// rest, on tiles, runs two iterations per pass (fgp2_iter_kernel) unless
+// opts.depth == 1 or the image is in FP32 or, by default, has
+// kFgp2dPassMaxPixels or more; an odd last iteration runs on the one-iteration
+// kernel.  P_j lives in buffer j mod nbuf (nbuf = 4 with two-iteration passes,
+// which write P_{k+1} and P_{k+2} while reading P_k and P_{k-1}; 3 otherwise).
 template <typename T, typename S>
 int fgp_solve(const T* d_f, T* d_out, T lambda, int iter, T epsil, int method, int nonneg, int nx, int ny, int nz,
               const Opts& opts, hipStream_t s, int* iters_done, float* re, const WarmState* ws) {

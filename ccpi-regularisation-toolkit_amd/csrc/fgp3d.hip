@@ -32,13 +32,14 @@ __device__ inline void orthogonal(float& v1, float& v2, float& v3, const float (
 // next plane's loads are issued a whole step ahead, and nothing else waits on
 // memory.
 //
-// Bound by HBM at large volumes (a pass reads 28 and writes 24 B per voxel at
-// about 4 TB/s: a region's rows start at any multiple of 4 B and the partial
-// lines of two regions meet; a copy of 64-aligned tiles of as many fields
-// reaches 5.2) and by VALU issue and barriers below: 256^3 111 -> 86 us per
-// iteration (bf16 90 -> 77, FP16 89 -> 75), 250^3 133 -> 80, 131 x 200 x 305
-// 66 -> 42, 128^3 19.6 -> 15.5 (bf16 17.2 -> 17.1, FP16 17.0 -> 15.8), 100^3
-// 13.9 -> 10.5 (before: two iterations per pass on 64 x 8 tiles, every stage
+// Bound by VALU issue, then by the traffic of overlapping regions: checked at
+// 256^3 (T = 4, 64 x 16 columns) the VALU instructions fill 82% of the CUs' busy
+// cycles at four each, and a launch reads 50 and writes 32 B per voxel at 3.1
+// TB/s where it needs 32 and 28 (a region loads each point 2.3 times, most of it
+// from L2, and the partial lines of two regions meet).  256^3 111 -> 86 us per
+// iteration (bf16 91 -> 76, FP16 89 -> 74), 250^3 133 -> 80, 300^3 221 -> 129, 131 x
+// 200 x 305 67 -> 43, 128^3 20.3 -> 16.0 (bf16 17.6 -> 16.6, FP16 17.4 -> 15.3), 100^3
+// 14.3 -> 10.2 (before: two iterations per pass on 64 x 8 tiles, every stage
 // through LDS).  T = 4 levels need 116-121 VGPRs: one 1024- or two 512-thread workgroups on a
 // CU.  Also measured: a level two planes behind the one before (one barrier
 // per plane for all levels, 15 instead of 8 values carried per row and level)
@@ -47,9 +48,9 @@ __device__ inline void orthogonal(float& v1, float& v2, float& v3, const float (
 //
 // DIR: FGP-dTV (top of dtv.hip).  R and the gradient of D are projected onto
 // the plane orthogonal to the reference's normalised gradient B, which travels
-// through the levels beside f; T = 3 fills the 128 VGPRs.  256^3 150 -> 120 us
-// per iteration, 300^3 322 -> 210, 190 x 257 x 231 156 -> 73, 160^3 45 -> 27,
-// 128^3 23.6 -> 19.6, 100^3 17.4 -> 13.0 (before: as for FGP).
+// through the levels beside f; T = 3 fills the 128 VGPRs.  256^3 152 -> 120 us
+// per iteration, 300^3 323 -> 189, 190 x 257 x 231 157 -> 74, 160^3 45 -> 29, 128^3
+// 24.1 -> 19.4, 100^3 17.8 -> 13.0 (before: as for FGP).
 template <class Sh, int T, typename S, bool ISO, bool CHK, bool DIR>
 __global__ __launch_bounds__(64 * Sh::NW, 4) void fgp_deep3_kernel(Fgp3Args a) {
     if (solve_stopped(a.ctrl)) return;
@@ -299,10 +300,10 @@ constexpr Deep3Cost kFgp3Cost16[kDeep3Shapes] = {
     {{1.7, 2.25, 2.85, 3.5}, {3.3, 3.3, 3.5, 3.6}},
 };
 
-// with B
+// with B (no pass has four levels)
 constexpr Deep3Cost kDtv3Cost[kDeep3Shapes] = {
-    {{2.4, 3.2, 4.05, 9.0}, {5.0, 5.0, 5.4, 9.0}},
-    {{2.1, 2.8, 3.25, 9.0}, {4.6, 4.6, 4.8, 9.0}},
+    {{2.4, 3.2, 4.05}, {5.0, 5.0, 5.4}},
+    {{2.1, 2.8, 3.25}, {4.6, 4.6, 4.8}},
 };
 
 template <typename S, bool DIR = false>

@@ -23,11 +23,12 @@ using Pd3Args = Deep3Args<4, Pd3Par>;
 //
 // Bound by VALU issue and the barriers (a step of four levels takes 3.5 us on
 // 16 waves whether its fields come from HBM or the last-level cache; about 115
-// VALU instructions per level and wave); with T <= 2 and FP32 P, by HBM.
-// 256^3 92 -> 73 us per iteration (bf16 89 -> 69, FP16 88 -> 67), 300^3 182 ->
-// 110 (175 -> 97), 190 x 257 x 231 83 -> 50 (80 -> 40), 160^3 29 -> 20, 128^3
-// 15.3 -> 14.6, 100^3 12.2 -> 10.2 (before: two iterations per pass on 64 x 8
-// tiles through LDS).
+// VALU instructions per level and wave; at 256^3 with T = 3 they fill 80% of the
+// CUs' busy cycles, and a launch moves 46 B per voxel of the 36 it needs at 3.3
+// TB/s); with T <= 2 and FP32 P, by HBM.  256^3 93 -> 73 us per iteration (bf16 90 ->
+// 66, FP16 89 -> 65), 300^3 183 -> 106 (bf16 178 -> 95), 190 x 257 x 231 84 -> 47 (81 ->
+// 40), 160^3 30 -> 20, 128^3 15.8 -> 15.3, 100^3 12.5 -> 10.3 (before: two iterations
+// per pass on 64 x 8 tiles through LDS).
 template <class Sh, int T, typename S, bool ISO, bool CHK>
 __global__ __launch_bounds__(64 * Sh::NW, 4) void pd_deep3_kernel(Pd3Args a) {
     if (solve_stopped(a.ctrl)) return;

@@ -202,7 +202,7 @@ struct Opts {
     int profile = 0;       // time each iteration with HIP events
     int wide_index = 0;    // force 64-bit element indexing
     int stream_launches = 0;  // batch: launch directly instead of one hipGraph
-    int depth = 0;         // iterations per pass where supported (FGP, PD, TGV 3D; FGP 2D below 2^20 pixels: 2 by default; 1 = off)
+    int depth = 0;         // iterations per pass: 0 as many as pay, 1 one, 2 two (register passes of volumes: as 0)
     int autotune = 0;      // choose tile_y / zchunk / depth by timing (tune.hip) when none is given
     int persistent = 0;    // batch: one persistent work-queue launch per group instead of per-level launches
     int tiled = 0;         // 3D FGP, PD: the tiled passes a group of jobs runs, not those in registers
@@ -213,10 +213,11 @@ struct Opts {
     size_t scratch_bytes = 0;
 };
 
-// 2D FGP runs two iterations per pass below this many pixels: there the
-// one-iteration kernel is launch/latency-bound (256^2: 6.5 -> 3.8 us per
-// iteration); from 1024^2 on the pass's ring evaluation costs more than the
-// traffic it saves (2048^2: 30.5 vs 32.3 us).
+// On tiles (FP64, grouped jobs) 2D FGP runs two iterations per pass below this
+// many pixels: there the one-iteration kernel is launch/latency-bound (256^2: 6.5
+// -> 3.8 us per iteration); from 1024^2 on the pass's ring evaluation costs more
+// than the traffic it saves (2048^2: 30.5 vs 32.3 us).  Under a scratch limit
+// larger FP32 images stay on tiles too, one iteration per launch.
 constexpr size_t kFgp2dPassMaxPixels = (size_t)1 << 20;
 
 // z planes per chunk of a grouped (batched / served) 3D job.
