@@ -226,8 +226,9 @@ int deep3_solve(M& m, const float* d_f, float* d_out, int nx, int ny, int nz, in
     if (ws)
         for (int i = 0; i < M::NF; ++i) m.store(i, ar.at(of[(q & 1) ^ 1][i]), *ws, n, s);
     if (last_iter) *last_iter = last;
-    CILREG_CK(hipGetLastError());
+    const hipError_t launched = hipGetLastError();
     CILREG_CK(hipStreamSynchronize(s));
+    CILREG_CK(launched);
     return 0;
 }
 

@@ -126,14 +126,16 @@ int free_idle_locked(int dev) {
 }
 }  // namespace
 
-// Failure injection for tests: the n-th next pool_alloc on this thread fails
-// as an exhausted device would (0 = off).
+// Failure injection for tests: the n-th next pool_alloc, or allocation of the
+// thread's pinned block, on this thread fails as an exhausted device would
+// (0 = off).
 static thread_local int g_fail_alloc_in = 0;
 
 void inject_alloc_failure(int n) { g_fail_alloc_in = n > 0 ? n : 0; }
+static bool alloc_fails() { return g_fail_alloc_in > 0 && --g_fail_alloc_in == 0; }
 
 void* pool_alloc(size_t bytes) {
-    if (g_fail_alloc_in > 0 && --g_fail_alloc_in == 0) return nullptr;
+    if (alloc_fails()) return nullptr;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
     std::lock_guard<std::mutex> lk(g_pool_mu);
@@ -248,7 +250,14 @@ struct PinnedSlot {
 
 int PinnedCtrl::allocate() {
     static thread_local PinnedSlot slot;
-    if (!slot.h) CILREG_CK(hipHostMalloc((void**)&slot.h, 2 * sizeof(Ctrl), hipHostMallocDefault));
+    if (!slot.h) {
+        if (alloc_fails() || hipHostMalloc((void**)&slot.h, 2 * sizeof(Ctrl), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            slot.h = nullptr;
+            set_error("pinned allocation of %zu bytes failed", 2 * sizeof(Ctrl));
+            return -1;
+        }
+    }
     h = slot.h;
     memset(h, 0, 2 * sizeof(Ctrl));
     return 0;

@@ -46,7 +46,8 @@ void pool_free(void* p);
 int pool_release_idle();
 // Bytes of the current device's pool held by running solves / kept idle.
 void pool_stats(size_t* busy, size_t* idle);
-// Test hook: the n-th next pool_alloc on this thread fails (0 = off).
+// Test hook: the n-th next pool_alloc, or allocation of the pinned block below,
+// on this thread fails (0 = off).
 void inject_alloc_failure(int n);
 // The drop-in host-pointer entry points free their device memory before
 // returning, as the reference's do, unless CILREG_KEEP_CACHE=1.
@@ -270,8 +271,9 @@ Geom plan_geom(K kernel, int threads, int nx, int ny, int nz, int ty, int zc_hin
 // The pass loop of every solve: pass(k, nk) launches the pass that advances
 // iterations k .. k+nk-1 (nk = width, fewer in the last pass) and returns what
 // fin needs to launch its finalisers.  Polls the stop flag every opts.poll
-// iterations without draining the queue; on return has synchronised the
-// stream and filled *iters_done and *re.  With opts.profile every pass is
+// iterations without draining the queue; on return, with an error too (the
+// caller's memory goes back to the pool), has synchronised the stream; fills
+// *iters_done and *re.  With opts.profile every pass is
 // timed with HIP events (the finalisers excluded); the profile reports time
 // per iteration (pass time / nk).
 template <class PassFn, class FinFn>
@@ -280,16 +282,16 @@ int drive_core(int iter, int width, float epsil, const Opts& opts, Ctrl* d_ctrl,
     PinnedCtrl pin;
     const bool use_tol = epsil != 0.0f;
     const bool polls = use_tol && !opts.scratch;   // an allocation-free solve does not poll
-    if (polls && pin.allocate() != 0) return -1;
+    int rc = polls ? pin.allocate() : 0;
     launch_ctrl_reset(d_ctrl, s);
     hipEvent_t ev[2] = {nullptr, nullptr};
     int flag_slot_pending[2] = {0, 0};
-    if (polls) {
-        CILREG_CK(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
-        CILREG_CK(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
-    }
+    for (int i = 0; i < 2 && polls && rc == 0; ++i)
+        if (hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) {
+            set_error("hipEventCreateWithFlags failed");
+            rc = -1;
+        }
     int poll_idx = 0, since_poll = 0;
-    int rc = 0;
     std::vector<hipEvent_t> pev;
     std::vector<int> pass_k, pass_n;
     if (opts.profile) {

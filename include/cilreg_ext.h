@@ -101,9 +101,10 @@ CILREG_API int cilreg_release_cache(void);
  * of the process hold memory. */
 CILREG_API int cilreg_pool_stats(size_t *busy_bytes, size_t *idle_bytes);
 
-/* Test hook for failure handling: the n-th next device allocation the
- * library requests on this host thread fails as an exhausted device would
- * (n = 0 turns it off).  Every entry point then returns -1 with the
+/* Test hook for failure handling: the n-th next allocation the library
+ * requests on this host thread (device memory, or the pinned block that a
+ * thread's first solve with a tolerance makes) fails as an exhausted device
+ * would (n = 0 turns it off).  Every entry point then returns -1 with the
  * allocation error and releases what it had allocated. */
 CILREG_API void cilreg_inject_alloc_failure(int n);
 

@@ -61,6 +61,60 @@ def test_dtv_allocates_once(shape):
     _same(got, want, f"{shape}")
 
 
+@pytest.mark.parametrize("case", ["dtv image", "dtv volume", "fgp volume on tiles", "tgv volume"])
+def test_failure_after_first_kernels_drains(case):
+    """A thread's first solve with a tolerance fails to get the pinned block it
+    polls through, after kernels that write its device memory were queued: it
+    returns with its stream drained, so the memory it hands back to the pool
+    is not written any more; the next solve succeeds."""
+    import ctypes
+    import threading
+    import torch
+    from ccpi.filters import device as D
+    from ccpi.filters.utils import require_gpu_lib
+    lib = require_gpu_lib()
+    lib.cilreg_inject_alloc_failure.argtypes = [ctypes.c_int]
+    lib.cilreg_inject_alloc_failure.restype = None
+    x = _vol((70, 90) if "image" in case else (60, 95, 100) if case == "dtv volume" else (20, 33, 67), 4)
+    ref = _vol(x.shape, 5)
+    big = torch.rand(4096, 4096, device="cuda")
+
+    def run():
+        if case.startswith("dtv"):
+            return D.dtv(x, ref, 0.03, 9, 1e-9)
+        return D.fgp(x, 0.03, 9, 1e-9) if case.startswith("fgp") else D.tgv(x, 0.03, 1.0, 2.0, 9, 12.0, 1e-9)
+
+    want = run()
+    torch.mm(big, big)
+    torch.cuda.synchronize()
+    res = {}
+
+    def first_of_a_thread():
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(60):
+                torch.mm(big, big)
+            res["busy"] = not s.query()
+            lib.cilreg_inject_alloc_failure(2)   # after the solve's device memory
+            try:
+                run()
+            except RuntimeError as e:
+                res["error"] = str(e)
+            finally:
+                lib.cilreg_inject_alloc_failure(0)
+            res["drained"] = s.query()
+            res["again"] = run()
+
+    t = threading.Thread(target=first_of_a_thread)
+    t.start()
+    t.join()
+    torch.cuda.synchronize()
+    assert res["busy"]
+    assert "alloc" in res.get("error", ""), res.get("error", "no error")
+    assert res["drained"], "the failed solve left work on its stream"
+    _same(res["again"], want, case)
+
+
 @pytest.mark.parametrize("rows", [1, 2, 3, 4, 5, 7, 8, 9])
 @pytest.mark.parametrize("method", ["fgp", "pd", "tgv", "rof", "sb", "ndf", "dtv"])
 def test_images_of_few_rows(method, rows):
